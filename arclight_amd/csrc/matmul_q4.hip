@@ -19,8 +19,8 @@
 // nibbles, the weights' offset of 8 folded into one multiply by the block's
 // value sum; lane sums meet in a DPP wave reduction.
 // Longer inputs (up to 64 tokens) take two launches: quantize_q8_kernel
-// (one thread per (token, block), into grow-only library scratch) and
-// gemv_q4_kernel (the same dot products, activations from that scratch).
+// (into grow-only library scratch, laid out as MFMA operands) and
+// gemm_q4_kernel, whose integer dot products run on the matrix cores.
 // Either way the 4-bit weights stream once: HBM-bound, 18 bytes per 32
 // weights.
 
@@ -37,45 +37,6 @@
 namespace {
 
 constexpr int kMaxT = 64;
-
-__global__ __launch_bounds__(256) void quantize_q8_kernel(const char * __restrict__ x, int64_t x_nb1, int K, int T,
-                                                          int8_t * __restrict__ qs, float * __restrict__ dx,
-                                                          int * __restrict__ sy) {
-    const int nb = K / 32;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= T * nb) return;
-    const int t = i / nb, b = i % nb;
-    const float4 * xb = (const float4 *) ((const float *) (x + (int64_t) t * x_nb1) + 32 * b);
-    float v[32];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float4 f = xb[j];
-        v[4 * j] = f.x; v[4 * j + 1] = f.y; v[4 * j + 2] = f.z; v[4 * j + 3] = f.w;
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) amax = fmaxf(amax, fabsf(v[j]));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    int sum = 0;
-    uint32_t words[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        uint32_t wv = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int q = (int) rintf(v[4 * j + k] * id);                 // ties to even, as vcvtnq
-            sum += q;
-            wv |= (uint32_t) (q & 0xff) << (8 * k);
-        }
-        words[j] = wv;
-    }
-    uint4 * out = (uint4 *) (qs + (int64_t) t * K + 32 * b);
-    out[0] = uint4{words[0], words[1], words[2], words[3]};
-    out[1] = uint4{words[4], words[5], words[6], words[7]};
-    dx[i] = (float) (_Float16) d;                                          // the block scale as stored (f16)
-    sy[i] = sum;
-}
 
 // Cross-lane moves on the VALU (DPP): within rows of 16 lanes, then the
 // broadcasts of a row's last lane into the next row(s).
@@ -114,54 +75,201 @@ __device__ __forceinline__ void block_of(const uint32_t (&c)[9 * BPL / 2], const
     }
 }
 
-template <int BPL>
-__global__ __launch_bounds__(256) void gemv_q4_kernel(const char * __restrict__ w, int64_t w_nb1, int N, int K,
-                                                      const int8_t * __restrict__ qs, const float * __restrict__ dx,
-                                                      const int * __restrict__ sy, int T, char * __restrict__ y,
-                                                      int64_t y_nb1) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= N) return;
-    const int nb = K / 32;
-    const int b0 = lane * BPL;
+// The four 16-lane groups' values of x (group d's in out[d], in all lanes).
+__device__ __forceinline__ void gather_groups(const float x, float (&out)[4]) {
+    const int xi = __builtin_bit_cast(int, x);
+    const auto h = __builtin_amdgcn_permlane32_swap(xi, xi, false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap((int) h[0], (int) h[0], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap((int) h[1], (int) h[1], false, false);
+    out[0] = __builtin_bit_cast(float, (int) a[0]);
+    out[1] = __builtin_bit_cast(float, (int) a[1]);
+    out[2] = __builtin_bit_cast(float, (int) b[0]);
+    out[3] = __builtin_bit_cast(float, (int) b[1]);
+}
+// q[d] of 16-lane group g <-> q[g] of group d (a 4 x 4 transpose).
+__device__ __forceinline__ void transpose_groups(uint32_t (&q)[4]) {
+    const auto a = __builtin_amdgcn_permlane32_swap((int) q[0], (int) q[2], false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap((int) q[1], (int) q[3], false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap((int) a[0], (int) b[0], false, false);
+    const auto d = __builtin_amdgcn_permlane16_swap((int) a[1], (int) b[1], false, false);
+    q[0] = (uint32_t) c[0]; q[1] = (uint32_t) c[1];
+    q[2] = (uint32_t) d[0]; q[3] = (uint32_t) d[1];
+}
 
-    // the lane's blocks of this row, 36-byte aligned in global memory
-    uint32_t c[9 * BPL / 2];
-    const uint32_t * wr = (const uint32_t *) (w + (int64_t) row * w_nb1 + (int64_t) b0 * 18);
+constexpr int min_c(int a, int b) { return a < b ? a : b; }
+constexpr int kTile = 16;                        // tokens of an MFMA tile
+constexpr int kGemmWaves = 8;                    // waves of a workgroup, each with 1/8 of K
+
+// Activations as gemm_q4_kernel's MFMA operands: one wavefront per (16-token
+// tile, pair of Q8_0 blocks), lane 16 g + t holding token t's values
+// 4g..4g+3 and 16+4g..16+4g+3 of both blocks (the nibble order of a Q4_0
+// dword), 16 bytes per lane, so operand loads and stores are whole 1 KiB
+// lines; the block scales (f16, as the format stores them) as
+// [tile][block][token]. Tokens past T are zeros.
+// Latency-bound (one load round; reads are whole 128-byte lines per token).
+__global__ __launch_bounds__(256) void quantize_q8_kernel(const char * __restrict__ x, int64_t x_nb1, int nb, int T,
+                                                          int n_items, uint4 * __restrict__ frag, _Float16 * __restrict__ dx) {
+    const int lane = threadIdx.x & 63;
+    const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (item >= n_items) return;
+    const int tile = item / (nb / 2), pair = item - tile * (nb / 2);
+    const int g = lane >> 4, tok = tile * kTile + (lane & 15);
+    float4 f[2][2] = {};
+    if (tok < T) {
+        const float * xr = (const float *) (x + (int64_t) tok * x_nb1) + 64 * pair + 4 * g;
 #pragma unroll
-    for (int i = 0; i < 9 * BPL / 2; ++i) c[i] = wr[i];
-    float dw[BPL];
-    uint32_t lo[BPL][4], hi[BPL][4];
-#pragma unroll
-    for (int j = 0; j < BPL; ++j) {
-        uint32_t q[4];
-        block_of<BPL>(c, j, dw[j], q);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            lo[j][i] = q[i] & 0x0f0f0f0fu;                             // values 4i .. 4i + 3
-            hi[j][i] = (q[i] >> 4) & 0x0f0f0f0fu;                      // values 16 + 4i ..
+        for (int k = 0; k < 2; ++k) {
+            f[k][0] = *(const float4 *) (xr + 32 * k);
+            f[k][1] = *(const float4 *) (xr + 32 * k + 16);
         }
     }
-
-    for (int t = 0; t < T; ++t) {
-        float part = 0.0f;
+    uint32_t words[4];
+    float d[2];
 #pragma unroll
-        for (int j = 0; j < BPL; ++j) {
-            const int b = b0 + j;
-            const uint4 * ab = (const uint4 *) (qs + (int64_t) t * K + 32 * b);
-            const uint4 a0 = ab[0], a1 = ab[1];
-            const uint32_t a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-            int dot = 0;
+    for (int k = 0; k < 2; ++k) {
+        const float v[8] = {f[k][0].x, f[k][0].y, f[k][0].z, f[k][0].w, f[k][1].x, f[k][1].y, f[k][1].z, f[k][1].w};
+        float amax = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                dot = __builtin_amdgcn_sdot4((int) lo[j][i], (int) a[i], dot, false);
-                dot = __builtin_amdgcn_sdot4((int) hi[j][i], (int) a[4 + i], dot, false);
-            }
-            const int sumi = dot - 8 * sy[t * nb + b];
-            part += ((float) sumi * dw[j]) * dx[t * nb + b];
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+        float gm[4];
+        gather_groups(amax, gm);
+        amax = fmaxf(fmaxf(gm[0], gm[1]), fmaxf(gm[2], gm[3]));
+        d[k] = amax / 127.0f;
+        const float id = d[k] != 0.0f ? 1.0f / d[k] : 0.0f;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            words[2 * k + w] = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)                                    // ties to even, as vcvtnq
+                words[2 * k + w] |= (uint32_t) ((int) rintf(v[4 * w + e] * id) & 0xff) << (8 * e);
         }
-        part = wave_sum_to_last(part);
-        if (lane == 63) *(float *) (y + (int64_t) t * y_nb1 + (int64_t) row * 4) = part;
+    }
+    frag[(int64_t) item * 64 + lane] = uint4{words[0], words[1], words[2], words[3]};
+    if (g < 2) dx[((int64_t) tile * nb + 2 * pair + g) * kTile + (lane & 15)] = (_Float16) (g ? d[1] : d[0]);
+}
+
+// 9 to 64 tokens: a workgroup takes 16 weight rows and a tile of 16 tokens,
+// each of its 8 waves 1/8 of K. One MFMA 16x16x32 i8 is one block's integer
+// dot products of 16 tokens and 16 rows, exact, as the format needs them;
+// its 4 results per lane then cost a conversion, a product and an FMA each.
+// That vector work and the unpacking (723 instructions per wave at K = 8192)
+// bound the kernel, so a workgroup takes one token tile: more would unpack
+// the weights once for several tiles, but leave CUs idle (K 8192, N 5120, 48
+// tokens: 21.4 us with one tile, 27.9 with three; 64 tokens: 25.7 with one,
+// 27.5 with two, 33.0 with four).
+// In a step the workgroup takes 64 blocks of every row, a wave 8: lanes 4 r
+// .. 4 r + 3 load row r's 144 bytes of them (a pair of blocks each), so that
+// a load touches few lines, and a permute brings row r's pair g to lane 16 g
+// + r (loaded there directly, 16 rows to a load's every quarter: 23.8
+// instead of 21.1 us). A block's MFMA operand wants dword g of it in group
+// g, which a transpose across the four groups gives for the four groups'
+// blocks together (4 permlane swaps). Nibbles become signed bytes of 16
+// times the weight (xor 8, shifted high), the 1/16 goes into the block scale
+// (both exact), so no sum of activations is needed. The activations come
+// straight from L2, 1 KiB per wave load, their scales through LDS (as vector
+// loads they took twice the operands' issue: 26.4 -> 24.0 us). The product of
+// two f16 scales is exact in f32, so a block adds one rounding; each block of
+// a step (at K = 4096 each pair) has a sum of its own and the waves' sums
+// meet in LDS in a tree, which keeps the error against the exact result at
+// that of one wave per row (2-norm 7.80e-8 at K = 8192, 7.37e-8 at 4096).
+// Measured, us per call with the quantization launch (before: one wave per
+// row, the tokens in series): K 8192, N 5120: 48 tokens 232 -> 21.9, 16
+// tokens 15.5; K 4096, N 2560: 37 tokens 39 -> 9.2, 16 tokens 22 -> 7.4; K
+// 4096, N 4096: 12 tokens 22 -> 7.5.
+template <int BL>
+__global__ __launch_bounds__(kGemmWaves * 64, 4) void gemm_q4_kernel(const char * w, int64_t w_nb1, int N, const uint4 * frag,
+                                                                  const uint4 * dx, int T, char * y, int64_t y_nb1) {
+    constexpr int NB = 32 * BL;                                        // blocks of a row
+    constexpr int kSteps = NB / (8 * kGemmWaves);
+    constexpr int kDx = NB * kTile * 2, kRed = kGemmWaves * 4 * 256;
+    __shared__ __align__(16) char lds[kDx > kRed ? kDx : kRed];        // the scales, then the waves' sums
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16, tile = blockIdx.y;
+    // the wave's blocks: 8 of every 64, group g's pair of those of step s
+    auto block = [&](const int s, const int d) { return (s * kGemmWaves + wave) * 8 + 2 * d; };
+    frag += (int64_t) tile * (NB / 2) * 64;
+    dx += (int64_t) tile * NB * 2;
+
+    // the wave's scales (it alone reads them: no barrier), 16-byte pieces
+    for (int i = lane; i < 16 * kSteps; i += 64) {
+        const int o = block(i >> 4, 0) * 2 + (i & 15);
+        ((uint4 *) lds)[o] = dx[o];
+    }
+    // A step's weights and operands go out together, kDepth steps ahead (a
+    // wave's loads return in order).
+    constexpr int kDepth = min_c(kSteps, 2);
+    uint32_t c[kDepth][9];
+    uint4 a[kDepth][4];
+    const char * wr = w + (int64_t) min(n0 + (lane >> 2), N - 1) * w_nb1;
+    auto issue = [&](const int s) {
+        const uint32_t * ws = (const uint32_t *) (wr + block(s, lane & 3) * 18);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) c[s % kDepth][i] = ws[i];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) a[s % kDepth][d] = frag[block(s, d) / 2 * 64 + lane];
+        asm volatile("" ::: "memory");                                 // keeps the issue order
+    };
+#pragma unroll
+    for (int s = 0; s < kDepth; ++s) issue(s);
+
+    typedef int int4v __attribute__((ext_vector_type(4)));
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    constexpr int kSums = kSteps > 2 ? 8 : 4;                          // sums a lane keeps per output: per block of a step, or pair
+    float acc[kSums / 4][4][4] = {};
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) {
+        uint32_t cs[9], q[2][4];
+        float dw[2][4];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) cs[i] = (uint32_t) __builtin_amdgcn_ds_bpermute(16 * r + 4 * g, (int) c[st % kDepth][i]);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            float d;
+            block_of<2>(cs, k, d, q[k]);
+            gather_groups(d * 0.0625f, dw[k]);
+            transpose_groups(q[k]);
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {                                  // the blocks of group d: b, b + 1
+            const int b = block(st, d);
+            const uint4 f = a[st % kDepth][d];
+            const long av[2] = {(long) ((uint64_t) f.x | (uint64_t) f.y << 32), (long) ((uint64_t) f.z | (uint64_t) f.w << 32)};
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const uint32_t x = q[k][d] ^ 0x88888888u;
+                const long wv = (long) ((uint64_t) ((x << 4) & 0xf0f0f0f0u) | (uint64_t) (x & 0xf0f0f0f0u) << 32);
+                const half4 s = *(const half4 *) (lds + ((b + k) * kTile + 4 * g) * 2);
+                const int4v sumi = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[k], wv, int4v{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[k % (kSums / 4)][d][i] = __builtin_fmaf((float) sumi[i], dw[k][d] * (float) s[i], acc[k % (kSums / 4)][d][i]);
+            }
+        }
+        if (st + kDepth < kSteps) issue(st + kDepth);
+    }
+    __syncthreads();                                                   // every wave is past its scales
+    float (*red)[4][64] = (float (*)[4][64]) lds;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float v[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) v[d] = kSums == 8 ? acc[0][d][i] + acc[kSums / 4 - 1][d][i] : acc[0][d][i];
+        red[wave][i][lane] = (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    __syncthreads();
+    // wave i < 4: token 4 (lane / 16) + i of the tile, row lane % 16
+    if (wave < 4) {
+        float v[kGemmWaves];
+#pragma unroll
+        for (int u = 0; u < kGemmWaves; ++u) v[u] = red[u][wave][lane];
+#pragma unroll
+        for (int h = kGemmWaves / 2; h >= 1; h /= 2)
+#pragma unroll
+            for (int u = 0; u < h; ++u) v[u] += v[u + h];
+        const int tok = tile * kTile + 4 * g + wave;
+        if (tok < T && n0 + r < N) *(float *) (y + (int64_t) tok * y_nb1 + (int64_t) (n0 + r) * 4) = v[0];
     }
 }
 
@@ -418,6 +526,16 @@ int launch_fused_t(const al_tensor * w, const al_tensor * x, const al_tensor * y
     return T == 1 ? launch_fused<BPL, 1>(w, x, y, N, K, T, st) : launch_fused<BPL, kFusedMaxT>(w, x, y, N, K, T, st);
 }
 
+template <int BL>
+int launch_gemm(const al_tensor * w, const al_tensor * y, int N, int tiles, int T, const uint4 * frag, const uint4 * dx,
+                hipStream_t st) {
+    const dim3 grid((unsigned) ((N + 15) / 16), (unsigned) tiles);
+    hipLaunchKernelGGL(gemm_q4_kernel<BL>, grid, dim3(kGemmWaves * 64), 0, st, (const char *) w->data, (int64_t) w->nb[1], N,
+                       frag, dx, T, (char *) y->data, (int64_t) y->nb[1]);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? AL_OK : al_hip_fail(e, "mul_mat_q4_0: launch");
+}
+
 // Per-device scratch for the quantized activations, grown on demand.
 struct Scratch {
     void * p = nullptr;
@@ -494,25 +612,23 @@ extern "C" int al_mul_mat_q4_0_f32(const al_tensor * w, const al_tensor * x, con
             default: return al_fail(AL_ERR_UNSUPPORTED, "mul_mat_q4_0: K %lld", (long long) K);
         }
     }
-    const size_t qs_bytes = (size_t) (T * K), f_bytes = (size_t) (T * nb) * 4;
+    const int tiles = (int) ((T + kTile - 1) / kTile);
+    const size_t qs_bytes = (size_t) tiles * kTile * (size_t) K, f_bytes = (size_t) tiles * kTile * (size_t) nb * 2;
     void * s = nullptr;
-    int rc = scratch(qs_bytes + 2 * f_bytes, &s);
+    int rc = scratch(qs_bytes + f_bytes, &s);
     if (rc != AL_OK) return rc;
-    int8_t * qs = (int8_t *) s;
-    float * dx = (float *) ((char *) s + qs_bytes);
-    int * sy = (int *) ((char *) s + qs_bytes + f_bytes);
-    hipLaunchKernelGGL(quantize_q8_kernel, dim3((unsigned) ((T * nb + 255) / 256)), dim3(256), 0, st,
-                       (const char *) x->data, (int64_t) x->nb[1], (int) K, (int) T, qs, dx, sy);
+    uint4 * frag = (uint4 *) s;
+    _Float16 * dx = (_Float16 *) ((char *) s + qs_bytes);
+    const int items = tiles * (int) (nb / 2);
+    hipLaunchKernelGGL(quantize_q8_kernel, dim3((unsigned) ((items + 3) / 4)), dim3(256), 0, st,
+                       (const char *) x->data, (int64_t) x->nb[1], (int) nb, (int) T, items, frag, dx);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return al_hip_fail(e, "mul_mat_q4_0: quantize launch");
-    const dim3 grid((unsigned) ((N + 3) / 4));
-    switch (nb / 64) {
-        case 2: hipLaunchKernelGGL(gemv_q4_kernel<2>, grid, dim3(256), 0, st, (const char *) w->data, (int64_t) w->nb[1], (int) N, (int) K, qs, dx, sy, (int) T, (char *) y->data, (int64_t) y->nb[1]); break;
-        case 4: hipLaunchKernelGGL(gemv_q4_kernel<4>, grid, dim3(256), 0, st, (const char *) w->data, (int64_t) w->nb[1], (int) N, (int) K, qs, dx, sy, (int) T, (char *) y->data, (int64_t) y->nb[1]); break;
-        case 6: hipLaunchKernelGGL(gemv_q4_kernel<6>, grid, dim3(256), 0, st, (const char *) w->data, (int64_t) w->nb[1], (int) N, (int) K, qs, dx, sy, (int) T, (char *) y->data, (int64_t) y->nb[1]); break;
-        case 8: hipLaunchKernelGGL(gemv_q4_kernel<8>, grid, dim3(256), 0, st, (const char *) w->data, (int64_t) w->nb[1], (int) N, (int) K, qs, dx, sy, (int) T, (char *) y->data, (int64_t) y->nb[1]); break;
+    switch (nb / 128) {
+        case 1: return launch_gemm<4>(w, y, (int) N, tiles, (int) T, frag, (const uint4 *) dx, st);
+        case 2: return launch_gemm<8>(w, y, (int) N, tiles, (int) T, frag, (const uint4 *) dx, st);
+        case 3: return launch_gemm<12>(w, y, (int) N, tiles, (int) T, frag, (const uint4 *) dx, st);
+        case 4: return launch_gemm<16>(w, y, (int) N, tiles, (int) T, frag, (const uint4 *) dx, st);
         default: return al_fail(AL_ERR_UNSUPPORTED, "mul_mat_q4_0: K %lld", (long long) K);
     }
-    e = hipGetLastError();
-    return e == hipSuccess ? AL_OK : al_hip_fail(e, "mul_mat_q4_0: launch");
 }

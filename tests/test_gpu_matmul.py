@@ -66,6 +66,27 @@ def test_wo_matches_oracle(gpu, K, N, T):
     assert rel < 1e-6, rel
 
 
+@pytest.mark.parametrize("K,N,T", [(4096, 15, 9), (4096, 17, 16), (8192, 16, 17), (8192, 2561, 33), (12288, 31, 48),
+                                   (16384, 33, 63)])
+def test_wo_token_tiles(gpu, K, N, T):
+    """More than 8 tokens (the matrix-core kernel): rows and tokens either
+    side of its 16 x 16 tiles, every K it is built for, padded rows of x and
+    y whose padding stays untouched, and weight scales of every sign,
+    denormal and zero. The bar is that of test_wo_matches_oracle."""
+    _case(f"wo tiles K={K} N={N} T={T}")
+    rng = np.random.default_rng(K + N * 5 + T)
+    w = O.random_q4_0(rng, N, K)
+    w["d"][:, ::7] ^= 0x8000                               # negative scales
+    w["d"][:, 3::11] = 5                                   # a denormal f16
+    w["d"][:, 5::13] = 0
+    x = _activations(rng, T, K)
+    got = _run(w, x, x_pad=8, y_pad=5)
+    want = O.mul_mat_q4_0(w, x)
+    bound = (K // 32 + 16) * 2 * EPS32 * abs_bound(dequant_q4_0(w), dequant_q8_0(O.quantize_q8_0(x)))
+    err = np.abs(got.astype(np.float64) - want)
+    assert np.all(err <= bound), f"worst {err.max():.3e} at {np.unravel_index((err - bound).argmax(), err.shape)}"
+
+
 @pytest.mark.parametrize("K,N,T", [(4096, 301, 1), (4096, 301, 2), (4096, 301, 8), (8192, 77, 5), (8192, 77, 9)])
 def test_wo_unit_scales_bit_exact(gpu, K, N, T):
     """Unit weight scales and activations whose every block has step 1:
