@@ -20,14 +20,15 @@ struct SetRowsParams {
 
 // Source row i of plane (i02, i03) converted to f16 (IEEE RNE) into cache
 // row idx[i]; an index out of range is not written but reported through
-// p.err. One workgroup of any size per row.
-__device__ __forceinline__ void set_rows_row(const SetRowsParams & p, const int i, const int i02, const int i03) {
+// p.err. Thread tid of n_threads takes every n_threads-th four values.
+__device__ __forceinline__ void set_rows_row(const SetRowsParams & p, const int i, const int i02, const int i03,
+                                             const int tid, const int n_threads) {
     const int i12 = i03 % p.i_ne2;
     const int i11 = i02 % p.i_ne1;
     const char * ip = p.idx + (int64_t) i * p.i_nb0 + (int64_t) i11 * p.i_nb1 + (int64_t) i12 * p.i_nb2;
     const int64_t i1 = p.idx64 ? *(const int64_t *) ip : (int64_t) *(const int32_t *) ip;
     if (i1 < 0 || i1 >= p.n_dst) {
-        if (threadIdx.x == 0) {
+        if (tid == 0) {
             if (atomicCAS(p.err, 0, 1) == 0) p.err[1] = (int) i1;
         }
         return;
@@ -35,14 +36,14 @@ __device__ __forceinline__ void set_rows_row(const SetRowsParams & p, const int 
     const float * src = (const float *) (p.src + (int64_t) i * p.s_nb1 + (int64_t) i02 * p.s_nb2 + (int64_t) i03 * p.s_nb3);
     _Float16 * dst = (_Float16 *) (p.dst + i1 * p.d_nb1 + (int64_t) i02 * p.d_nb2 + (int64_t) i03 * p.d_nb3);
     if (p.vec4) {
-        for (int c = 4 * threadIdx.x; c < p.nc; c += 4 * blockDim.x) {
+        for (int c = 4 * tid; c < p.nc; c += 4 * n_threads) {
             const float4 x = *(const float4 *) (src + c);
             typedef _Float16 half4 __attribute__((ext_vector_type(4)));
             half4 h = {(_Float16) x.x, (_Float16) x.y, (_Float16) x.z, (_Float16) x.w};
             *(half4 *) (dst + c) = h;
         }
     } else {
-        for (int c = threadIdx.x; c < p.nc; c += blockDim.x) dst[c] = (_Float16) src[c];
+        for (int c = tid; c < p.nc; c += n_threads) dst[c] = (_Float16) src[c];
     }
 }
 

@@ -1,5 +1,5 @@
-// Per-head RMSNorm, weight and rotary embedding of one 128-float row by one
-// wavefront (gfx950): the arithmetic of the attention-input producers,
+// Per-head RMSNorm, weight and rotary embedding of 128-float rows, 8 lanes
+// to a row (gfx950): the arithmetic of the attention-input producers,
 // shared by the stand-alone kernels and the decode kernel that folds them
 // into its prologue, so that both give the same bits.
 //   rms_norm  nnml/src/ops/ops.cpp:680-726
@@ -16,18 +16,45 @@ struct RopeConsts {
     float theta_scale, freq_scale, ext_factor, corr0, corr1, mscale;
 };
 
-__device__ __forceinline__ double norm_rope_wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+// Dims of pair i. MODE: 0 no rotation, 1 pairs (2i, 2i + 1), 2 NEOX pairs
+// (i, i + 64).
+template <int MODE> __device__ __forceinline__ int rope_d0(const int i) { return MODE == 1 ? 2 * i : i; }
+template <int MODE> __device__ __forceinline__ int rope_d1(const int i) { return MODE == 1 ? 2 * i + 1 : i + 64; }
+
+// The sum of v over groups of 8 lanes, in every lane of the group (DPP:
+// lanes within a quad, then the two quads of 8 lanes mirrored).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(const double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) (uint32_t) b, CTRL, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t) __builtin_amdgcn_update_dpp(0, (int) (uint32_t) (b >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, (uint64_t) lo | (uint64_t) hi << 32);
+}
+__device__ __forceinline__ double sum8(double v) {
+    v += dpp_move<0xb1>(v);                      // quad_perm [1, 0, 3, 2]
+    v += dpp_move<0x4e>(v);                      // quad_perm [2, 3, 0, 1]
+    v += dpp_move<0x141>(v);                     // row_half_mirror
     return v;
 }
 
-// Dims of the lane's pair. MODE: 0 no rotation, 1 pairs (2i, 2i + 1),
-// 2 NEOX pairs (i, i + 64).
-template <int MODE> __device__ __forceinline__ int rope_d0(const int lane) { return MODE == 1 ? 2 * lane : lane; }
-template <int MODE> __device__ __forceinline__ int rope_d1(const int lane) { return MODE == 1 ? 2 * lane + 1 : lane + 64; }
+// x of lane l times scale, l times over, each product rounded: step k runs
+// with the lanes above k enabled, one vector instruction a step (as selects
+// the 63 steps were three each). Needs all 64 lanes of the wave.
+__device__ __forceinline__ void rope_angle_steps(float & x, const float scale) {
+    uint64_t all;
+    asm volatile("s_mov_b64 %1, exec\n\t"
+                 ".rept 63\n\t"
+                 "s_lshl_b64 exec, exec, 1\n\t"
+                 "v_mul_f32 %0, %2, %0\n\t"
+                 ".endr\n\t"
+                 "s_mov_b64 exec, %1"
+                 : "+v"(x), "=&s"(all)
+                 : "s"(scale)
+                 : "scc");
+}
 
-// cos / sin (times mscale) of the lane's pair at position pos (ops.cpp:743-772).
+// cos / sin (times mscale) of the lane's pair at position pos (ops.cpp:743-772);
+// every lane of the wave takes part.
 template <int MODE>
 __device__ __forceinline__ void rope_cos_sin(const RopeConsts & r, const int32_t pos, const int lane, float & c,
                                              float & s) {
@@ -38,10 +65,8 @@ __device__ __forceinline__ void rope_cos_sin(const RopeConsts & r, const int32_t
     c = 1.0f;
     s = 0.0f;
     if constexpr (MODE != 0) {
-        const float theta_extrap0 = (float) pos;
-        float theta_extrap = theta_extrap0;
-        for (int k = 0; k < 63; ++k)
-            if (k < lane) theta_extrap *= r.theta_scale;
+        float theta_extrap = (float) pos;
+        rope_angle_steps(theta_extrap, r.theta_scale);
         const float theta_interp = r.freq_scale * theta_extrap;
         float theta = theta_interp;
         if (r.ext_factor != 0.0f) {
@@ -50,34 +75,9 @@ __device__ __forceinline__ void rope_cos_sin(const RopeConsts & r, const int32_t
             const float mix = ramp * r.ext_factor;
             theta = theta_interp * (1.0f - mix) + theta_extrap * mix;
         }
-        c = cosf(theta) * r.mscale;
-        s = sinf(theta) * r.mscale;
-    }
-}
-
-// y = rope(rms_norm(x) * w) at dims d0, d1 of the lane, given the pair's
-// cos / sin (rope_cos_sin): x0, x1 and w0, w1 are those dims of the row and
-// of the weight (has_w false: no weight); every lane of the wave takes part
-// (the norm's sum is a wave reduction).
-template <int MODE>
-__device__ __forceinline__ void norm_rope_apply(const float x0, const float x1, const bool has_w, const float w0,
-                                                const float w1, const float eps, const float c, const float s,
-                                                float & y0, float & y1) {
-#pragma clang fp contract(off)
-    const float sq0 = x0 * x0, sq1 = x1 * x1;
-    const double sum = norm_rope_wave_sum((double) sq0 + (double) sq1);
-    const float mean = (float) (sum / 128.0);
-    const float scale = 1.0f / sqrtf(mean + eps);
-    float n0 = x0 * scale, n1 = x1 * scale;
-    if (has_w) {
-        n0 = n0 * w0;
-        n1 = n1 * w1;
-    }
-    y0 = n0;
-    y1 = n1;
-    if constexpr (MODE != 0) {
-        y0 = n0 * c - n1 * s;
-        y1 = n0 * s + n1 * c;
+        sincosf(theta, &s, &c);
+        c *= r.mscale;
+        s *= r.mscale;
     }
 }
 
@@ -85,11 +85,11 @@ __device__ __forceinline__ void norm_rope_apply(const float x0, const float x1, 
 // 8i..8i+7 of a wave hold one row), each lane with 8 rotation pairs: lo[k]
 // and hi[k] are the two dims of the lane's pair k, w_lo / w_hi their
 // weights (1 where there is no weight, which leaves the product bit for bit
-// unchanged), rot[k] the pair's (cos, sin). Per value the arithmetic of
-// norm_rope_apply; the row's sum of squares (double) is added in another
-// order, so the two can differ only where the partial sums are not exact in
+// unchanged), rot[k] the pair's (cos, sin). The row's sum of squares is
+// taken in double; which pairs a lane holds decides the order of its terms,
+// so two layouts can differ only where the partial sums are not exact in
 // double, by rounding in the double's last bits, far below the f32 mean's
-// resolution. Every lane of the wave takes part (the sum's shuffles).
+// resolution. Every lane of the wave takes part (the sum's moves).
 template <int MODE>
 __device__ __forceinline__ void norm_rope_group8(const float (&lo)[8], const float (&hi)[8], const float (&w_lo)[8],
                                                  const float (&w_hi)[8], const float eps, const float2 (&rot)[8],
@@ -105,10 +105,7 @@ __device__ __forceinline__ void norm_rope_group8(const float (&lo)[8], const flo
     for (int h = 4; h >= 1; h /= 2)
 #pragma unroll
         for (int k = 0; k < h; ++k) part[k] += part[k + h];
-    double sum = part[0];
-    sum += __shfl_xor(sum, 1);
-    sum += __shfl_xor(sum, 2);
-    sum += __shfl_xor(sum, 4);
+    const double sum = sum8(part[0]);
     const float mean = (float) (sum / 128.0);
     const float scale = 1.0f / sqrtf(mean + eps);
 #pragma unroll
@@ -121,14 +118,4 @@ __device__ __forceinline__ void norm_rope_group8(const float (&lo)[8], const flo
             y_hi[k] = n0 * rot[k].y + n1 * rot[k].x;
         }
     }
-}
-
-// Both steps for one row.
-template <int MODE>
-__device__ __forceinline__ void norm_rope_pair(const float x0, const float x1, const bool has_w, const float w0,
-                                               const float w1, const float eps, const RopeConsts & r,
-                                               const int32_t pos, const int lane, float & y0, float & y1) {
-    float c, s;
-    rope_cos_sin<MODE>(r, pos, lane, c, s);
-    norm_rope_apply<MODE>(x0, x1, has_w, w0, w1, eps, c, s, y0, y1);
 }

@@ -9,14 +9,20 @@
 // multiplied i times by theta_scale in float, exactly as the cache loop
 // carries it.
 //
-// One wavefront per (token, head) row of 128 floats: lane l holds the two
-// elements of rotation pair l (dims l and l + 64 for NEOX, 2l and 2l + 1
-// otherwise), so the norm is one wave reduction and the rotation needs no
-// data exchange. A workgroup takes 4 heads of one token; the pair angles and
-// their cos / sin are computed once per wave.
+// One wavefront takes 8 heads of one token, 8 lanes to a row of 128 floats:
+// lane j of 8 holds dims 4j..4j+3 of each 32, so that a load or store of the
+// wave covers whole 128-byte lines; the norm's sum is three DPP moves, and a
+// row's rotation needs no other lane's values. The rotation's 64 (cos, sin)
+// pairs are computed one per lane, once for the 8 rows, and handed over
+// through LDS within the wave.
+//
+// What bounds it: for many tokens memory, for few the chain position ->
+// angle (63 products in series) -> sine -> rows. One row per wave repeated
+// that chain for every row and was bound by its vector instructions.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -36,23 +42,69 @@ struct NormRopeParams {
     const char * rows;  int64_t rows_nb0;          // cache rows [T] or null
     int32_t rows64;
     int64_t n_rows_dst;
+    int32_t y_vec;                                 // cache rows 8-byte aligned
     int32_t H, T;
     float eps;
     RopeConsts rope;
     int * err;                                     // [2]: first out-of-range cache row
 };
 
-// Row (head h, token t), one wavefront. MODE: 0 no rotation, 1 pairs
-// (2i, 2i + 1), 2 NEOX pairs (i, i + 64).
+constexpr int kRows = 8;                         // rows of a wave: heads of one token
+constexpr int kWaves = 4;                        // waves of a workgroup: tokens
+
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+
+// Rows of heads h0 .. h0 + 7 of token t, one wavefront; rot: the wave's 64
+// (cos, sin) pairs in LDS. MODE: 0 no rotation, 1 pairs (2i, 2i + 1), 2 NEOX
+// pairs (i, i + 64).
 template <int MODE, bool CACHE>
-__device__ __forceinline__ void norm_rope_row(const NormRopeParams & p, const int h, const int t, const int lane) {
-    if (h >= p.H) return;
-    const int d0 = rope_d0<MODE>(lane), d1 = rope_d1<MODE>(lane);
-    const float w0 = p.w ? p.w[d0] : 1.0f;
-    const float w1 = p.w ? p.w[d1] : 1.0f;
-    const float * xr = (const float *) (p.x + (int64_t) h * p.x_nb1 + (int64_t) t * p.x_nb2);
-    float y0, y1;
-    norm_rope_pair<MODE>(xr[d0], xr[d1], p.w != nullptr, w0, w1, p.eps, p.rope, MODE != 0 ? p.pos[t] : 0, lane, y0, y1);
+__device__ __forceinline__ void norm_rope_rows(const NormRopeParams & p, const int h0, const int t, const int lane,
+                                               float2 * rot) {
+    if (h0 >= p.H) return;
+    const int l8 = lane & 7, h = h0 + (lane >> 3);
+    const float * xr = (const float *) (p.x + (int64_t) min(h, p.H - 1) * p.x_nb1 + (int64_t) t * p.x_nb2);
+    float4u x[4], w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = *(const float4u *) (xr + 32 * j + 4 * l8);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = p.w ? *(const float4u *) (p.w + 32 * j + 4 * l8) : float4u{1.0f, 1.0f, 1.0f, 1.0f};
+    // pair k of the lane: in place (k % 4) of piece k / 4 and of the piece 64
+    // dims on, or (MODE 1) values 2 (k % 2), 2 (k % 2) + 1 of piece k / 2
+    float lo[8], hi[8], wl[8], wh[8];
+    float2 cs[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int j = MODE == 1 ? k / 2 : k / 4, e = MODE == 1 ? 2 * (k % 2) : k % 4;
+        lo[k] = x[j][e];
+        hi[k] = MODE == 1 ? x[j][e + 1] : x[j + 2][e];
+        wl[k] = w[j][e];
+        wh[k] = MODE == 1 ? w[j][e + 1] : w[j + 2][e];
+    }
+    if constexpr (MODE != 0) {
+        float c, s;
+        rope_cos_sin<MODE>(p.rope, p.pos[t], lane, c, s);
+        rot[lane] = float2{c, s};
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < 8; k += 2) {
+            const int first = MODE == 1 ? 16 * (k / 2) + 2 * l8 : 32 * (k / 4) + 4 * l8 + k % 4;   // its pair
+            const float4 v = *(const float4 *) (rot + first);
+            cs[k] = float2{v.x, v.y};
+            cs[k + 1] = float2{v.z, v.w};
+        }
+    }
+    float yl[8], yh[8];
+    norm_rope_group8<MODE>(lo, hi, wl, wh, p.eps, cs, yl, yh);
+    float4u y[4];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int j = MODE == 1 ? k / 2 : k / 4, e = MODE == 1 ? 2 * (k % 2) : k % 4;
+        y[j][e] = yl[k];
+        if constexpr (MODE == 1) y[j][e + 1] = yh[k];
+        else y[j + 2][e] = yh[k];
+    }
     if constexpr (CACHE) {
         const char * ip = p.rows + (int64_t) t * p.rows_nb0;
         const int64_t r = p.rows64 ? *(const int64_t *) ip : (int64_t) *(const int32_t *) ip;
@@ -60,41 +112,62 @@ __device__ __forceinline__ void norm_rope_row(const NormRopeParams & p, const in
             if (lane == 0 && atomicCAS(p.err, 0, 1) == 0) p.err[1] = (int) r;
             return;
         }
+        if (h >= p.H) return;
         _Float16 * yr = (_Float16 *) (p.y + r * p.y_nb1) + (int64_t) h * 128;
-        yr[d0] = (_Float16) y0;
-        yr[d1] = (_Float16) y1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const half4 v = {(_Float16) y[j][0], (_Float16) y[j][1], (_Float16) y[j][2], (_Float16) y[j][3]};
+            _Float16 * d = yr + 32 * j + 4 * l8;
+            if (p.y_vec) {
+                *(half4 *) d = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[e] = v[e];
+            }
+        }
     } else {
+        if (h >= p.H) return;
         float * yr = (float *) (p.y + (int64_t) h * p.y_nb1 + (int64_t) t * p.y_nb2);
-        yr[d0] = y0;
-        yr[d1] = y1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(float4u *) (yr + 32 * j + 4 * l8) = y[j];
     }
 }
 
 template <int MODE, bool CACHE>
-__global__ __launch_bounds__(256) void norm_rope_kernel(const NormRopeParams p) {
+__global__ __launch_bounds__(64 * kWaves) void norm_rope_kernel(const NormRopeParams p) {
+    __shared__ __attribute__((aligned(16))) float2 rot[kWaves][64];
     prefetch_params(p);
-    norm_rope_row<MODE, CACHE>(p, blockIdx.y * 4 + (threadIdx.x >> 6), blockIdx.x, threadIdx.x & 63);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.x * kWaves + wave;
+    if (t < p.T) norm_rope_rows<MODE, CACHE>(p, blockIdx.y * kRows, t, threadIdx.x & 63, rot[wave]);
 }
 
 // The attention inputs of one layer in one launch: blockIdx.y < yq are Q
-// rows (4 heads per workgroup), then yk of K rows into the cache, then one
-// workgroup per token for its V row.
+// rows, then yk of K rows into the cache, then yv of the tokens' V rows.
+// Traced, us per launch, one row per wave before: 512 tokens of 32 + 8 heads
+// 14.3 -> 5.3, 1024 tokens of 64 + 8 heads 41.5 -> 13.2 (5.9 TB/s), 4 tokens
+// of 32 + 8 heads 3.7 -> 2.5.
 template <int MODE>
-__global__ __launch_bounds__(256) void attn_inputs_kernel(const NormRopeParams q, const NormRopeParams k,
-                                                          const SetRowsParams v, const int yq, const int yk) {
-    prefetch_params(q, k, v, yq, yk);
+__global__ __launch_bounds__(64 * kWaves) void attn_inputs_kernel(const NormRopeParams q, const NormRopeParams k,
+                                                                  const SetRowsParams v, const int yq, const int yk,
+                                                                  const int yv) {
+    __shared__ __attribute__((aligned(16))) float2 rot[kWaves][64];
+    prefetch_params(q, k, v, yq, yk, yv);
     const int by = blockIdx.y;
-    const int hw = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (by < yq) norm_rope_row<MODE, false>(q, by * 4 + hw, blockIdx.x, lane);
-    else if (by < yq + yk) norm_rope_row<MODE, true>(k, (by - yq) * 4 + hw, blockIdx.x, lane);
-    else set_rows_row(v, blockIdx.x, 0, 0);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.x * kWaves + wave;
+    if (t >= q.T) return;
+    if (by < yq) norm_rope_rows<MODE, false>(q, by * kRows, t, lane, rot[wave]);
+    else if (by < yq + yk) norm_rope_rows<MODE, true>(k, (by - yq) * kRows, t, lane, rot[wave]);
+    else set_rows_row(v, t, 0, 0, (by - yq - yk) * 64 + lane, yv * 64);
 }
 
 template <int MODE>
 hipError_t launch_mode(const NormRopeParams & p, bool cache, hipStream_t stream) {
-    const dim3 grid((unsigned) p.T, (unsigned) ((p.H + 3) / 4));
-    if (cache) hipLaunchKernelGGL((norm_rope_kernel<MODE, true>), grid, dim3(256), 0, stream, p);
-    else       hipLaunchKernelGGL((norm_rope_kernel<MODE, false>), grid, dim3(256), 0, stream, p);
+    const dim3 grid((unsigned) ((p.T + kWaves - 1) / kWaves), (unsigned) ((p.H + kRows - 1) / kRows));
+    if (cache) hipLaunchKernelGGL((norm_rope_kernel<MODE, true>), grid, dim3(64 * kWaves), 0, stream, p);
+    else       hipLaunchKernelGGL((norm_rope_kernel<MODE, false>), grid, dim3(64 * kWaves), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -163,6 +236,7 @@ int norm_rope_params(const al_tensor * x, const al_tensor * w, const al_tensor *
         p.y_nb2 = (int64_t) y->nb[2];
     }
     p.y = (char *) y->data;
+    p.y_vec = (((uintptr_t) p.y | (uintptr_t) p.y_nb1) & 7u) == 0;
     if (!p.x || !p.y) return al_fail(AL_ERR_INVALID, "rms_norm_rope: null data");
     *out = p;
     *mode_out = mode;
@@ -250,13 +324,15 @@ extern "C" int al_attn_inputs_f32(const al_attn_inputs_args * a, void * stream) 
     rc = set_rows_params(&a->v_cache, &a->v, &a->rows, &v, &empty);
     if (rc != AL_OK) return rc;
     if (empty) return al_fail(AL_ERR_INVALID, "attn_inputs: empty v");
-    const int yq = (q.H + 3) / 4, yk = (k.H + 3) / 4;
-    const dim3 grid((unsigned) q.T, (unsigned) (yq + yk + 1));
+    // V: 256 values of a row to a wave (one load each lane), at most 8 waves
+    const int yq = (q.H + kRows - 1) / kRows, yk = (k.H + kRows - 1) / kRows;
+    const int yv = std::max(1, std::min(8, (v.nc + 255) / 256));
+    const dim3 grid((unsigned) ((q.T + kWaves - 1) / kWaves), (unsigned) (yq + yk + yv));
     hipStream_t s = (hipStream_t) stream;
     switch (mq) {
-        case 2: hipLaunchKernelGGL(attn_inputs_kernel<2>, grid, dim3(256), 0, s, q, k, v, yq, yk); break;
-        case 1: hipLaunchKernelGGL(attn_inputs_kernel<1>, grid, dim3(256), 0, s, q, k, v, yq, yk); break;
-        default: hipLaunchKernelGGL(attn_inputs_kernel<0>, grid, dim3(256), 0, s, q, k, v, yq, yk); break;
+        case 2: hipLaunchKernelGGL(attn_inputs_kernel<2>, grid, dim3(64 * kWaves), 0, s, q, k, v, yq, yk, yv); break;
+        case 1: hipLaunchKernelGGL(attn_inputs_kernel<1>, grid, dim3(64 * kWaves), 0, s, q, k, v, yq, yk, yv); break;
+        default: hipLaunchKernelGGL(attn_inputs_kernel<0>, grid, dim3(64 * kWaves), 0, s, q, k, v, yq, yk, yv); break;
     }
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AL_OK : al_hip_fail(e, "attn_inputs: launch");

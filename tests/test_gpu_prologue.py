@@ -209,3 +209,42 @@ def test_attn_inputs_bad_row_reported(gpu):
     fattn.device_errors()                                  # cleared
     assert kc.numpy(np.uint16)[3].any() and vc.numpy(np.uint16)[3].any()
     assert not np.delete(kc.numpy(np.uint16), 3, axis=0).any() and not np.delete(vc.numpy(np.uint16), 3, axis=0).any()
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,mode", [(1, 1, 1, abi.AL_ROPE_NEOX), (5, 9, 3, abi.AL_ROPE_NORMAL), (4, 16, 17, None),
+                                           (13, 7, 8, abi.AL_ROPE_NEOX)])
+def test_attn_inputs_row_and_token_groups(gpu, T, Hq, Hkv, mode):
+    """Heads and tokens either side of the 8 rows of a wave and the 4 waves of
+    a workgroup, rows at 4-byte aligned addresses and cache rows at odd
+    strides, against the oracle (the bars of this file); nothing outside the
+    tokens' rows is written."""
+    from arclight_amd import device, fattn, prologue
+    _case(f"attention inputs T={T} heads {Hq} + {Hkv} mode={mode}, unaligned rows")
+    rng = np.random.default_rng(T + Hq)
+    n_rows, rope = 40, abi.AlRopeParams(128, mode, 40960, 1e6, 1.0, 0.0, 1.0, 32.0, 1.0) if mode is not None else None
+    x, wq, pos = _inputs(90 + T, T, Hq + Hkv)
+    wk = rng.standard_normal(128).astype(np.float32)
+    v = (rng.standard_normal((T, Hkv * 128)) * 3).astype(np.float32)
+    rows = rng.choice(n_rows, T, replace=False).astype(np.int64)
+    row = (Hq + Hkv) * 512 + 4                             # a token's row of x, then one float of padding
+    flat = np.zeros((T, row // 4), np.float32)
+    flat[:, 1:] = x.reshape(T, -1)
+    buf = device.DeviceTensor.from_numpy(flat).buf
+    q = device.DeviceTensor(buf, abi.AL_TYPE_F32, (T, Hq, 128), (row, 512, 4), 4)
+    k = device.DeviceTensor(buf, abi.AL_TYPE_F32, (T, Hkv, 128), (row, 512, 4), 4 + Hq * 512)
+    store = [device.DeviceTensor.from_numpy(np.zeros((n_rows, Hkv * 128 + 1), np.uint16)) for _ in range(2)]
+    cache = [device.DeviceTensor(s.buf, abi.AL_TYPE_F16, (n_rows, Hkv * 128), (Hkv * 256 + 2, 2), 0) for s in store]
+    d = {n: device.DeviceTensor.from_numpy(a) for n, a in (("v", v), ("wq", wq), ("wk", wk), ("pos", pos), ("rows", rows))}
+    q_out = device.DeviceTensor.empty((T, Hq, 128), np.float32)
+    prologue.attn_inputs(q, d["wq"], k, d["wk"], d["v"], d["pos"], d["rows"], q_out, cache[0], cache[1], eps=EPS, rope=rope)
+    device.synchronize()
+    fattn.device_errors()
+    ref_q = O.rms_norm_rope(np.ascontiguousarray(x[:, :Hq]), wq, pos, eps=EPS, rope=rope)
+    np.testing.assert_allclose(q_out.numpy(np.float32), ref_q, rtol=1e-6, atol=1e-5)
+    ref_k = O.rms_norm_rope(np.ascontiguousarray(x[:, Hq:]), wk, pos, eps=EPS, rope=rope).reshape(T, -1)
+    got_k, got_v = (s.numpy(np.uint16) for s in store)
+    ulp = np.abs(got_k[rows, :-1].astype(np.int32) - ref_k.astype(np.float16).view(np.uint16).astype(np.int32))
+    assert ulp.max() <= 1
+    assert np.array_equal(got_v[rows, :-1], v.astype(np.float16).view(np.uint16))
+    for got in (got_k, got_v):
+        assert not got[:, -1].any() and not np.delete(got, rows, axis=0).any()
