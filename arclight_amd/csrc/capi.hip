@@ -141,7 +141,9 @@ static int library_workspace(size_t bytes, void * stream, void ** ptr) {
             w.ptr = nullptr;
             w.bytes = 0;
         }
-        const size_t sz = std::max(bytes, (size_t) 4 << 20);
+        // room for any prefill call (at most one 128-row record a CU) and any
+        // one-stream decode call, so that those never grow it
+        const size_t sz = std::max(bytes, (size_t) 20 << 20);
         hipError_t e = hipMalloc(&w.ptr, sz);
         if (e != hipSuccess) return al_fail(AL_ERR_HIP, "hipMalloc(workspace %zu bytes): %s", sz, hipGetErrorString(e));
         e = hipMemset(w.ptr, 0, sz);
@@ -189,6 +191,7 @@ struct Plan {
     int rows_per_tile = 16;
     size_t part_offset = 0;         // merge records: workspace offset and bytes (0: none)
     size_t part_bytes = 0;
+    size_t scratch_floor = 0;       // a caller's scratch below this is refused
     size_t workspace_bytes() const { return part_bytes ? part_offset + part_bytes : 0; }
 };
 
@@ -240,6 +243,20 @@ int prefill_max_split() {
 int prefill_split_tiles() {
     static int v = env_int("AL_PREFILL_SPLIT_TILES", 4);
     return v;
+}
+
+// Time of a prefill launch in us, as measured over chunks of 256 to 1024
+// tokens and 512 to 24576 cells (32 and 64 heads, 8 kv heads): a workgroup
+// fills a CU and takes 7 us plus 1.0 (128 rows) or 1.08 us (64 rows, two
+// tiles at a time) per iteration over its cell tiles; workgroups past the
+// CUs wait for a round; with more than one to a row tile the last to arrive
+// loads all their records. So 64 rows against 128 rows in twice the splits
+// changes sides at about 50 iterations (512 tokens of 32 heads: 48.1 against
+// 49.9 us at 3584 cells, 89.6 against 87.0 at 8192, 261 against 221 at 24576).
+double prefill_cost(int rows, int64_t split, int64_t units, int64_t iterations, int n_cu) {
+    const int64_t rounds = (units * split + n_cu - 1) / n_cu;
+    const double merge = split > 1 ? 1.5 + (double) (rows * split) / 96.0 : 0.0;
+    return (double) rounds * (7.0 + (rows == kFattnPrefillRows ? 1.0 : 1.08) * (double) iterations) + merge;
 }
 
 int wgs_per_cu() {
@@ -325,10 +342,32 @@ int decode_max_split() {
     return v;
 }
 
+// Scratch of prefill row tiles shared by split > 1 workgroups.
+size_t prefill_scratch(int rows, int64_t split, int64_t units) {
+    return kFattnCounterBytes + (size_t) (units * split * rows) * kFattnRecordStride * sizeof(float);
+}
+
+// The least scratch a caller has to bring to a prefill call (less is refused,
+// not run slower): that of row tiles of 128 rows, or of 64 where 128 leave
+// CUs idle, shared by just enough workgroups to fill the device.
+size_t prefill_scratch_floor(int64_t R, int64_t heads, int64_t cell_tiles, int n_cu) {
+    const int rows = prefill_rows_forced() ? prefill_rows_forced()
+                     : (R + kFattnPrefillRows - 1) / kFattnPrefillRows * heads >= n_cu ? kFattnPrefillRows
+                                                                                       : kFattnPrefillRows / 2;
+    const int64_t units = (R + rows - 1) / rows * heads;
+    int64_t split = 1;
+    while (split < prefill_max_split() && units * split < n_cu &&
+           cell_tiles >= prefill_split_tiles() * (kFattnPrefillRows / rows) * (split + 1))
+        ++split;
+    return split > 1 ? prefill_scratch(rows, split, units) : 0;
+}
+
 // Mirrors the asserts of nnml_flash_attn_ext (nnml/src/tensor.cpp:1292-1320)
 // and nnml_compute_forward_flash_attn_ext_f16 (arm.cpp:2213-2245), then the
 // limits of this path.
-int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, Plan * out) {
+// ws_bytes: the scratch at hand; where a plan can do with less (prefill row
+// tiles shared by fewer workgroups), it asks for no more.
+int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_bytes, Plan * out) {
     if (!a) return al_fail(AL_ERR_INVALID, "fattn: null arguments");
     const al_tensor &q = a->q, &k = a->k, &v = a->v, &m = a->mask, &s = a->sinks, &d = a->dst;
     if (!q.data || !k.data || !v.data || !d.data) return al_fail(AL_ERR_INVALID, "fattn: q, k, v and dst are required");
@@ -416,27 +455,38 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, Plan * out) 
     p.m0 = powf(2.0f, -(p.max_bias) / p.n_head_log2);
     p.m1 = powf(2.0f, -(p.max_bias / 2.0f) / p.n_head_log2);
 
-    // Many query rows: the prefill kernel, one workgroup per row tile of 128
-    // rows, or of 64 rows (two cell splits inside the workgroup) when
-    // 128-row tiles leave CUs idle; n_split workgroups per tile (each taking
-    // every n_split-th share of the 64-cell tiles of the visible range) when
-    // the row tiles alone still do not fill the device. It keeps the running
-    // max on scores as computed, so it needs scale > 0 unless softcapped.
-    const int64_t big_units = (p.R + kFattnPrefillRows - 1) / kFattnPrefillRows * Hkv * B;
-    const int prefill_rows = prefill_rows_forced() ? prefill_rows_forced()
-                             : big_units >= n_cu ? kFattnPrefillRows : kFattnPrefillRows / 2;
+    // Many query rows: the prefill kernel, row tiles of 128 rows, or of 64
+    // rows (two cell splits inside the workgroup), each shared by n_split
+    // workgroups that take every n_split-th share of the visible range's
+    // 64-cell tiles: whichever prefill_cost() holds cheapest, splits only
+    // while every workgroup has a CU (520 tokens of 64 heads over 2000 cells:
+    // 73 us unsplit, 81 in three). It keeps the running max on scores as
+    // computed, so it needs scale > 0 unless softcapped.
+    int64_t prefill_extent = p.kv_hi;
+    if (p.causal_pos0 >= 0) prefill_extent = std::min<int64_t>(prefill_extent, p.causal_pos0 + T);
+    const int64_t cell_tiles = std::max<int64_t>(1, (prefill_extent + 63) / 64);
+    int prefill_rows = 0;
+    int64_t prefill_split = 1;
+    double best = 0.0;
+    for (int rows = kFattnPrefillRows; rows >= kFattnPrefillRows / 2; rows /= 2) {
+        if (prefill_rows_forced() && rows != prefill_rows_forced()) continue;
+        const int in_wg = kFattnPrefillRows / rows;
+        const int64_t units = (p.R + rows - 1) / rows * Hkv * B;
+        for (int64_t split = 1; split <= prefill_max_split(); ++split) {
+            if (split > 1 && (units * split > n_cu || cell_tiles < prefill_split_tiles() * in_wg * split ||
+                              prefill_scratch(rows, split, units) > ws_bytes))
+                break;
+            const double c = prefill_cost(rows, split, units, (cell_tiles + split * in_wg - 1) / (split * in_wg), n_cu);
+            if (!prefill_rows || c < best) {
+                prefill_rows = rows;
+                prefill_split = split;
+                best = c;
+            }
+        }
+    }
     const int in_wg_split = kFattnPrefillRows / prefill_rows;
     const int64_t prefill_tiles = (p.R + prefill_rows - 1) / prefill_rows;
     const int64_t prefill_units = prefill_tiles * Hkv * B;
-    int64_t prefill_split = 1;
-    {
-        int64_t extent = p.kv_hi;
-        if (p.causal_pos0 >= 0) extent = std::min<int64_t>(extent, p.causal_pos0 + T);
-        const int64_t cell_tiles = std::max<int64_t>(1, (extent + 63) / 64);
-        while (prefill_split < prefill_max_split() && prefill_units * prefill_split < n_cu &&
-               cell_tiles >= prefill_split_tiles() * in_wg_split * (prefill_split + 1))
-            ++prefill_split;
-    }
     // (an explicit mask: the prefill kernel reads its rows 16 bytes at a time)
     const bool mask_rows16 = !m.data || (aligned16(m.data) && m.nb[1] % 16 == 0 && m.nb[2] % 16 == 0 && m.nb[3] % 16 == 0);
     const bool prefill_shape = !p.dyn && p.R >= prefill_min_rows() && prefill_units <= kFattnCounterWords &&
@@ -445,11 +495,9 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, Plan * out) 
                                (uint64_t) (n_kv + 64) * v.nb[1] + 256 <= (uint64_t) UINT32_MAX && mask_rows16 &&
                                lds_per_block >= (int64_t) fattn_prefill_lds_bytes() && q_slice < INT32_MAX &&
                                (p.softcap != 0.0f || p.scale > 0.0f) && prefer_prefill();
-    const size_t prefill_part = prefill_split > 1 ? (size_t) prefill_units * prefill_split * prefill_rows *
-                                                        kFattnRecordStride * sizeof(float)
-                                                  : 0;
     if (prefill_shape) {
         pl.kernel = kPrefill;
+        pl.scratch_floor = prefill_scratch_floor(p.R, Hkv * B, cell_tiles, n_cu);
         pl.rows_per_tile = prefill_rows;
         p.n_row_tiles = (int32_t) prefill_tiles;
         p.n_split = (int32_t) prefill_split;
@@ -458,7 +506,7 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, Plan * out) 
         p.tiles_magic = magic_u32(prefill_tiles);
         if (prefill_split > 1) {
             pl.part_offset = kFattnCounterBytes;
-            pl.part_bytes = prefill_part;
+            pl.part_bytes = prefill_scratch(prefill_rows, prefill_split, prefill_units) - kFattnCounterBytes;
         }
         *out = pl;
         return AL_OK;
@@ -575,7 +623,7 @@ extern "C" uint64_t al_fattn_workspace_bytes(const al_fattn_args * a) {
     int n_cu = 0, lds = 0;
     if (al_device_cu_count(&n_cu) != AL_OK || al_device_lds_per_block(&lds) != AL_OK) return 0;
     Plan pl;
-    if (make_plan(a, n_cu, lds, &pl) != AL_OK) return 0;
+    if (make_plan(a, n_cu, lds, UINT64_MAX, &pl) != AL_OK) return 0;
     return pl.workspace_bytes();
 }
 
@@ -592,13 +640,13 @@ static int fattn_run(const al_fattn_args * a, void * noalloc_ws, size_t noalloc_
     if (rc == AL_OK) rc = al_device_lds_per_block(&lds);
     if (rc != AL_OK) return rc;
     Plan pl;
-    rc = make_plan(a, n_cu, lds, &pl);
+    rc = make_plan(a, n_cu, lds, noalloc_ws ? noalloc_bytes : a && a->workspace ? a->workspace_bytes : UINT64_MAX, &pl);
     if (rc != AL_OK) return rc;
     if (fused && (pl.kernel != kDecode || !fattn_decode_fused_ok(pl.waves, pl.stages) || pl.p.R > 16 ||
                   pl.p.B != 1 || pl.p.mask))
         return al_fail(AL_ERR_UNSUPPORTED, "fattn_with_inputs: the call does not run on the decode kernel "
                        "(up to 16 rows per kv head, one stream, no mask tensor)");
-    const size_t need = pl.workspace_bytes();
+    const size_t need = std::max(pl.workspace_bytes(), pl.scratch_floor);
     if (need) {
         void * ws = noalloc_ws ? noalloc_ws : a->workspace;
         if (noalloc_ws) {

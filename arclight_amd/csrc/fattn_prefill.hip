@@ -70,6 +70,7 @@ using namespace fattn_prefill;
 
 constexpr int kTC = 64;                          // cells per tile
 constexpr int kTileBytes = kTC * 256;            // one tile of K or of V (16 KiB)
+constexpr int kRotWindow = 8;                    // iterations the row tiles' first tiles are staggered over
 static_assert(kLds == 10 * kTileBytes, "10 tiles fill the LDS");
 static_assert(80 * 1024 + 128 * 512 + 128 * 8 <= kLds - 16 && 64 * kFattnRecordStride * 4 <= 80 * 1024,
               "output staging fits past the merge records");
@@ -272,13 +273,19 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     const int n_all = p.n_split * S::SP;
     const int s_all = sx * S::SP + si;
     const int NT = (max(hi_wg, 0) + kTC - 1) / kTC;
-    // NI = ceil(NT / n_all) and rot ~ rt NI / n_row_tiles by multiply-high
-    // with the plan's reciprocals (0: divisor 1); rot only staggers the
-    // splits' first tiles, so its rounding only needs rot < NI
+    // NI = ceil(NT / n_all) and rot ~ rt min(NI, kRotWindow) / n_row_tiles by
+    // multiply-high with the plan's reciprocals (0: divisor 1); rot only
+    // staggers the row tiles' first tiles, so its rounding only needs rot <
+    // NI. The window keeps the row tiles of a head, which run on one XCD,
+    // within 8 iterations of each other, so that they share the tiles in its
+    // L2: spread over all of a long context each streamed the whole K/V from
+    // beyond it (us per layer, 512 tokens over 24576 cells: 64 rows a tile 478
+    // -> 261, 128 rows 245 -> 221; 256 tokens over 16384 cells 164 -> 94). No
+    // stagger at all is 4 % slower at 1536 cells.
     const int NI = __builtin_amdgcn_readfirstlane(
         p.split_magic ? (int) __umulhi((uint32_t) (NT + n_all - 1), p.split_magic) : NT);
     const int rot = __builtin_amdgcn_readfirstlane(
-        NI > 0 ? min((int) __umulhi((uint32_t) (rt * NI), p.tiles_magic), NI - 1) : 0);
+        NI > 0 ? min((int) __umulhi((uint32_t) (rt * min(NI, kRotWindow)), p.tiles_magic), NI - 1) : 0);
     const int n_vis = max(min(hi_wg, p.n_kv), 1);
     auto tile_c0 = [&](const int i) {                     // branch-free: selects only
         int j = i + rot;

@@ -252,6 +252,31 @@ def test_prefill_kernel_chunk512_qwen3_4b(gpu, pos0):
     _check(f"prefill chunk 512 pos0 {pos0}", q, k, v, scale=SCALE, kv_len=pos0 + 512, causal_pos0=pos0)
 
 
+def test_prefill_row_tiles_by_context_and_scratch(gpu):
+    """A 512-token chunk over a long context runs 128-row tiles in two
+    workgroups each; with less scratch at hand (but what a shared tile of
+    such a call ever needed) it runs unshared tiles, and takes 64-row tiles
+    over a short one. Causal and with a mask tensor, against the oracle."""
+    from arclight_amd import device, fattn
+    n_kv = 7168
+    q, k, v = O.make_inputs(530, T=512, Hq=32, Hkv=8, n_kv=n_kv)
+    dq, dk, dv = fattn.upload_q(q), fattn.upload_kv(k), fattn.upload_kv(v)
+    dst = device.DeviceTensor.empty(q.shape, np.float32, axes=abi.DST_AXES)
+    ref = O.attention(q, k, v, scale=SCALE, kv_len=n_kv, causal_pos0=n_kv - 512)
+    need = fattn.workspace_bytes(dq, dk, dv, None, None, dst, scale=SCALE, kv_len=n_kv, causal_pos0=n_kv - 512)
+    assert need >= 128 * 2 * 128 * 528                     # records of 128 rows, two workgroups to each of 128 tiles
+    assert fattn.workspace_bytes(dq, dk, dv, None, None, dst, scale=SCALE, kv_len=1024, causal_pos0=512) == 0
+    for nbytes in (need, need - 4, 1 << 20):
+        _case(f"prefill 512 tokens over {n_kv} cells, {nbytes} bytes of scratch")
+        ws = device.DeviceBuffer(nbytes)
+        ws.zero()
+        fattn.flash_attn_ext(dq, dk, dv, scale=SCALE, kv_len=n_kv, causal_pos0=n_kv - 512, dst=dst, workspace=ws)
+        device.synchronize()
+        assert_parity(dst.numpy(np.float32), ref, what=f"{nbytes} bytes of scratch")
+    m = O.causal_mask(512, n_kv, n_kv - 600, kv_len=n_kv - 88)
+    _check("prefill 512 tokens, long mask tensor", q, k, v, m, scale=SCALE)
+
+
 def test_prefill_kernel_gqa8_noncausal_sinks_softcap(gpu):
     rng = np.random.default_rng(8)
     q, k, v = O.make_inputs(600, T=256, Hq=64, Hkv=8, n_kv=1000)
