@@ -192,7 +192,7 @@ struct Plan {
     size_t part_offset = 0;         // merge records: workspace offset and bytes (0: none)
     size_t part_bytes = 0;
     size_t scratch_floor = 0;       // a caller's scratch below this is refused
-    size_t workspace_bytes() const { return part_bytes ? part_offset + part_bytes : 0; }
+    size_t workspace_bytes() const { return std::max(part_bytes ? part_offset + part_bytes : 0, scratch_floor); }
 };
 
 bool aligned16(const void * ptr) { return ((uintptr_t) ptr & 15u) == 0; }
@@ -218,9 +218,16 @@ int env_int(const char * name, int dflt) {
 }
 
 // Fewest query rows per kv head that go to the prefill kernel
-// (AL_PREFILL_MIN_ROWS); fewer take the decode or split-KV kernel.
+// (AL_PREFILL_MIN_ROWS); fewer take the decode kernel. Below
+// kMaskedPrefillRows with a mask tensor the split-KV kernel is kept: the
+// prefill kernel reads a mask that is no causal prefix (several sequences in
+// one cache) value by value. Measured, us per layer with the inputs, split-KV
+// against prefill: 9 tokens of 32 heads over 500 cells 31.5 / 12.9, over 8000
+// 43.9 / 25.3, 37 over 3000 66 / 19, 63 over 8000 95 / 28; 16 sequences in
+// one cache of 16384 cells 89 / 150.
+constexpr int kMaskedPrefillRows = 256;
 int prefill_min_rows() {
-    static int v = env_int("AL_PREFILL_MIN_ROWS", 256);
+    static int v = env_int("AL_PREFILL_MIN_ROWS", 33);
     return v;
 }
 
@@ -349,7 +356,8 @@ size_t prefill_scratch(int rows, int64_t split, int64_t units) {
 
 // The least scratch a caller has to bring to a prefill call (less is refused,
 // not run slower): that of row tiles of 128 rows, or of 64 where 128 leave
-// CUs idle, shared by just enough workgroups to fill the device.
+// CUs idle, shared by just enough workgroups to fill the device (below
+// kMaskedPrefillRows rows: that of the split-KV kernel).
 size_t prefill_scratch_floor(int64_t R, int64_t heads, int64_t cell_tiles, int n_cu) {
     const int rows = prefill_rows_forced() ? prefill_rows_forced()
                      : (R + kFattnPrefillRows - 1) / kFattnPrefillRows * heads >= n_cu ? kFattnPrefillRows
@@ -360,6 +368,33 @@ size_t prefill_scratch_floor(int64_t R, int64_t heads, int64_t cell_tiles, int n
            cell_tiles >= prefill_split_tiles() * (kFattnPrefillRows / rows) * (split + 1))
         ++split;
     return split > 1 ? prefill_scratch(rows, split, units) : 0;
+}
+
+// Sizes of the split-KV kernel for the call in pl->p.
+void splitkv_plan(Plan * pl, int n_cu) {
+    FattnParams & p = pl->p;
+    pl->rows_per_tile = fattn_splitkv_rows_per_tile(std::min(p.R, 64));
+    p.n_row_tiles = (p.R + pl->rows_per_tile - 1) / pl->rows_per_tile;
+    int64_t extent = p.kv_hi;
+    if (p.causal_pos0 >= 0) extent = std::min<int64_t>(extent, p.causal_pos0 + p.T);
+    extent = std::max<int64_t>(extent, 0);
+    const int64_t tiles = (extent + 31) / 32;
+    const int64_t units = (int64_t) p.Hkv * p.n_row_tiles * p.B;
+    const int64_t waves = fattn_splitkv_waves(pl->rows_per_tile);
+    const int64_t target = (int64_t) n_cu * wgs_per_cu();
+    int64_t n_split = (target + units - 1) / units;
+    // every wave of a split gets at least one 32-cell tile
+    n_split = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(n_split, (tiles + waves - 1) / waves), kFattnMaxSplit));
+    int64_t cps_tiles = std::max<int64_t>(1, (tiles + n_split - 1) / n_split);
+    p.cells_per_split = (int32_t) (cps_tiles * 32);
+    n_split = std::max<int64_t>(1, (extent + p.cells_per_split - 1) / p.cells_per_split);
+    if (units > kFattnCounterWords) n_split = 1;
+    if (n_split == 1) p.cells_per_split = (int32_t) std::max<int64_t>(32, (extent + 31) / 32 * 32);
+    p.n_split = (int32_t) n_split;
+    if (p.n_split > 1) {
+        pl->part_offset = kFattnCounterBytes;
+        pl->part_bytes = (size_t) units * p.n_split * pl->rows_per_tile * kFattnRecordStride * sizeof(float);
+    }
 }
 
 // Mirrors the asserts of nnml_flash_attn_ext (nnml/src/tensor.cpp:1292-1320)
@@ -489,7 +524,7 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
     const int64_t prefill_units = prefill_tiles * Hkv * B;
     // (an explicit mask: the prefill kernel reads its rows 16 bytes at a time)
     const bool mask_rows16 = !m.data || (aligned16(m.data) && m.nb[1] % 16 == 0 && m.nb[2] % 16 == 0 && m.nb[3] % 16 == 0);
-    const bool prefill_shape = !p.dyn && p.R >= prefill_min_rows() && prefill_units <= kFattnCounterWords &&
+    const bool prefill_shape = !p.dyn && p.R >= (m.data ? kMaskedPrefillRows : prefill_min_rows()) && prefill_units <= kFattnCounterWords &&
                                (uint64_t) p.R * (uint64_t) p.G < (1ull << 32) && prefill_tiles * B <= 65535 &&
                                (uint64_t) (n_kv + 64) * k.nb[1] + 256 <= (uint64_t) UINT32_MAX &&
                                (uint64_t) (n_kv + 64) * v.nb[1] + 256 <= (uint64_t) UINT32_MAX && mask_rows16 &&
@@ -497,7 +532,13 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
                                (p.softcap != 0.0f || p.scale > 0.0f) && prefer_prefill();
     if (prefill_shape) {
         pl.kernel = kPrefill;
-        pl.scratch_floor = prefill_scratch_floor(p.R, Hkv * B, cell_tiles, n_cu);
+        if (p.R >= kMaskedPrefillRows) {
+            pl.scratch_floor = prefill_scratch_floor(p.R, Hkv * B, cell_tiles, n_cu);
+        } else {
+            Plan sk = pl;
+            splitkv_plan(&sk, n_cu);
+            pl.scratch_floor = sk.workspace_bytes();
+        }
         pl.rows_per_tile = prefill_rows;
         p.n_row_tiles = (int32_t) prefill_tiles;
         p.n_split = (int32_t) prefill_split;
@@ -590,29 +631,7 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
     if (p.dyn)
         return al_fail(AL_ERR_UNSUPPORTED, "fattn: dyn_len needs the decode kernel (up to 32 query rows per kv head)");
 
-    // split-KV sizing
-    pl.rows_per_tile = fattn_splitkv_rows_per_tile(std::min(p.R, 64));
-    p.n_row_tiles = (p.R + pl.rows_per_tile - 1) / pl.rows_per_tile;
-    int64_t extent = p.kv_hi;
-    if (p.causal_pos0 >= 0) extent = std::min<int64_t>(extent, p.causal_pos0 + T);
-    extent = std::max<int64_t>(extent, 0);
-    const int64_t tiles = (extent + 31) / 32;
-    const int64_t units = (int64_t) Hkv * p.n_row_tiles * B;
-    const int64_t waves = fattn_splitkv_waves(pl.rows_per_tile);
-    const int64_t target = (int64_t) n_cu * wgs_per_cu();
-    int64_t n_split = (target + units - 1) / units;
-    // every wave of a split gets at least one 32-cell tile
-    n_split = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(n_split, (tiles + waves - 1) / waves), kFattnMaxSplit));
-    int64_t cps_tiles = std::max<int64_t>(1, (tiles + n_split - 1) / n_split);
-    p.cells_per_split = (int32_t) (cps_tiles * 32);
-    n_split = std::max<int64_t>(1, (extent + p.cells_per_split - 1) / p.cells_per_split);
-    if (units > kFattnCounterWords) n_split = 1;
-    if (n_split == 1) p.cells_per_split = (int32_t) std::max<int64_t>(32, (extent + 31) / 32 * 32);
-    p.n_split = (int32_t) n_split;
-    if (p.n_split > 1) {
-        pl.part_offset = kFattnCounterBytes;
-        pl.part_bytes = (size_t) units * p.n_split * pl.rows_per_tile * kFattnRecordStride * sizeof(float);
-    }
+    splitkv_plan(&pl, n_cu);
     *out = pl;
     return AL_OK;
 }
@@ -646,7 +665,7 @@ static int fattn_run(const al_fattn_args * a, void * noalloc_ws, size_t noalloc_
                   pl.p.B != 1 || pl.p.mask))
         return al_fail(AL_ERR_UNSUPPORTED, "fattn_with_inputs: the call does not run on the decode kernel "
                        "(up to 16 rows per kv head, one stream, no mask tensor)");
-    const size_t need = std::max(pl.workspace_bytes(), pl.scratch_floor);
+    const size_t need = pl.workspace_bytes();
     if (need) {
         void * ws = noalloc_ws ? noalloc_ws : a->workspace;
         if (noalloc_ws) {

@@ -277,6 +277,20 @@ def test_prefill_row_tiles_by_context_and_scratch(gpu):
     _check("prefill 512 tokens, long mask tensor", q, k, v, m, scale=SCALE)
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,n_kv,pos0", [(33, 1, 1, 40, 0), (9, 32, 8, 17, 8), (16, 32, 8, 4096, 4000),
+                                                (17, 32, 8, 3000, 2983), (63, 32, 8, 500, 437), (31, 64, 8, 2048, 1900),
+                                                (51, 10, 2, 700, 100)])
+def test_few_rows_on_the_prefill_kernel(gpu, T, Hq, Hkv, n_kv, pos0):
+    """33 to 255 query rows per kv head without a mask tensor: one row, one
+    tile and one cell either side of its 64-row tiles, causal and not, with
+    sinks and softcap, and in two streams."""
+    q, k, v = O.make_inputs(7000 + T, B=2 if Hkv == 2 else 1, T=T, Hq=Hq, Hkv=Hkv, n_kv=n_kv)
+    name = f"{T} tokens of {Hq} heads over {n_kv} cells"
+    _check(f"{name}, causal from {pos0}", q, k, v, scale=SCALE, kv_len=min(n_kv, pos0 + T), causal_pos0=pos0)
+    sinks = np.random.default_rng(T).standard_normal(Hq).astype(np.float32)
+    _check(f"{name}, sinks + softcap", q, k, v, None, sinks, scale=SCALE * 3, logit_softcap=4.0, kv_len=n_kv - 1)
+
+
 def test_prefill_kernel_gqa8_noncausal_sinks_softcap(gpu):
     rng = np.random.default_rng(8)
     q, k, v = O.make_inputs(600, T=256, Hq=64, Hkv=8, n_kv=1000)
