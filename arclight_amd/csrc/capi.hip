@@ -218,14 +218,11 @@ int env_int(const char * name, int dflt) {
 }
 
 // Fewest query rows per kv head that go to the prefill kernel
-// (AL_PREFILL_MIN_ROWS); fewer take the decode kernel. Below
-// kMaskedPrefillRows with a mask tensor the split-KV kernel is kept: the
-// prefill kernel reads a mask that is no causal prefix (several sequences in
-// one cache) value by value. Measured, us per layer with the inputs, split-KV
-// against prefill: 9 tokens of 32 heads over 500 cells 31.5 / 12.9, over 8000
-// 43.9 / 25.3, 37 over 3000 66 / 19, 63 over 8000 95 / 28; 16 sequences in
-// one cache of 16384 cells 89 / 150.
-constexpr int kMaskedPrefillRows = 256;
+// (AL_PREFILL_MIN_ROWS); fewer take the decode kernel. Measured, us per layer
+// with the inputs, split-KV against prefill: 9 tokens of 32 heads over 500
+// cells 31.5 / 12.9, over 8000 43.9 / 17.6, 37 over 3000 66 / 17.9, 63 over 8000
+// 95 / 25; with a mask tensor 37 over 3000
+// 83 / 25, 16 sequences in one cache of 16384 cells 89 / 35.
 int prefill_min_rows() {
     static int v = env_int("AL_PREFILL_MIN_ROWS", 33);
     return v;
@@ -242,28 +239,33 @@ int prefill_rows_forced() {
 
 // Prefill workgroup splits: at most AL_PREFILL_MAX_SPLIT per row tile, and a
 // split only when each workgroup keeps at least AL_PREFILL_SPLIT_TILES 64-cell
-// tiles per in-workgroup split.
+// tiles per in-workgroup split (2 against 4, us per layer: 16 tokens over 3000
+// cells 16.2 / 18.2, 100 over 1000 17.2 / 18.4).
 int prefill_max_split() {
     static int v = std::min(env_int("AL_PREFILL_MAX_SPLIT", kFattnPrefillMaxSplit), kFattnPrefillMaxSplit);
     return v;
 }
 int prefill_split_tiles() {
-    static int v = env_int("AL_PREFILL_SPLIT_TILES", 4);
+    static int v = env_int("AL_PREFILL_SPLIT_TILES", 2);
     return v;
 }
 
-// Time of a prefill launch in us, as measured over chunks of 256 to 1024
-// tokens and 512 to 24576 cells (32 and 64 heads, 8 kv heads): a workgroup
+// Time of a prefill launch in us, as measured over chunks of 9 to 1024
+// tokens and 200 to 24576 cells (32 and 64 heads, 8 kv heads): a workgroup
 // fills a CU and takes 7 us plus 1.0 (128 rows) or 1.08 us (64 rows, two
-// tiles at a time) per iteration over its cell tiles; workgroups past the
-// CUs wait for a round; with more than one to a row tile the last to arrive
-// loads all their records. So 64 rows against 128 rows in twice the splits
-// changes sides at about 50 iterations (512 tokens of 32 heads: 48.1 against
-// 49.9 us at 3584 cells, 89.6 against 87.0 at 8192, 261 against 221 at 24576).
-double prefill_cost(int rows, int64_t split, int64_t units, int64_t iterations, int n_cu) {
+// tiles at a time) per iteration over its cell tiles, 2.4 when it takes a
+// mask value by value; workgroups past the CUs wait for a round. With more
+// than one to a row tile the last to arrive loads all their records, or,
+// above four, several share that behind the split flags. So 64 rows against
+// 128 rows in twice the splits changes sides at about 50 iterations (512
+// tokens of 32 heads: 48.1 against 49.9 us at 3584 cells, 89.6 against 87.0 at
+// 8192, 261 against 221 at 24576), and few row tiles over a long cache go to
+// as many workgroups as there are CUs (9 tokens over 8000 cells: 25.6 us in 4,
+// 19.1 in 8, 17.6 in 32; 16 sequences in one cache of 16384 cells 96 / 58 / 35).
+double prefill_cost(int rows, int64_t split, int64_t units, int64_t iterations, int n_cu, bool by_value) {
     const int64_t rounds = (units * split + n_cu - 1) / n_cu;
-    const double merge = split > 1 ? 1.5 + (double) (rows * split) / 96.0 : 0.0;
-    return (double) rounds * (7.0 + (rows == kFattnPrefillRows ? 1.0 : 1.08) * (double) iterations) + merge;
+    const double merge = split == 1 ? 0.0 : split > 4 ? 4.0 : 1.5 + (double) (rows * split) / 96.0;
+    return (double) rounds * (7.0 + (by_value ? 2.4 : rows == kFattnPrefillRows ? 1.0 : 1.08) * (double) iterations) + merge;
 }
 
 int wgs_per_cu() {
@@ -357,15 +359,16 @@ size_t prefill_scratch(int rows, int64_t split, int64_t units) {
 // The least scratch a caller has to bring to a prefill call (less is refused,
 // not run slower): that of row tiles of 128 rows, or of 64 where 128 leave
 // CUs idle, shared by just enough workgroups to fill the device (below
-// kMaskedPrefillRows rows: that of the split-KV kernel).
+// kManyRows rows: that of the split-KV kernel).
+constexpr int kManyRows = 256;
 size_t prefill_scratch_floor(int64_t R, int64_t heads, int64_t cell_tiles, int n_cu) {
     const int rows = prefill_rows_forced() ? prefill_rows_forced()
                      : (R + kFattnPrefillRows - 1) / kFattnPrefillRows * heads >= n_cu ? kFattnPrefillRows
                                                                                        : kFattnPrefillRows / 2;
     const int64_t units = (R + rows - 1) / rows * heads;
     int64_t split = 1;
-    while (split < prefill_max_split() && units * split < n_cu &&
-           cell_tiles >= prefill_split_tiles() * (kFattnPrefillRows / rows) * (split + 1))
+    while (split < std::min(prefill_max_split(), 4) && units * split < n_cu &&
+           cell_tiles >= 4 * (kFattnPrefillRows / rows) * (split + 1))
         ++split;
     return split > 1 ? prefill_scratch(rows, split, units) : 0;
 }
@@ -500,6 +503,12 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
     int64_t prefill_extent = p.kv_hi;
     if (p.causal_pos0 >= 0) prefill_extent = std::min<int64_t>(prefill_extent, p.causal_pos0 + T);
     const int64_t cell_tiles = std::max<int64_t>(1, (prefill_extent + 63) / 64);
+    // A mask over few rows is as a rule that of several sequences in one
+    // cache, which the kernel takes value by value, with less work to a split
+    // (9 sequences of up to 200 cells: 30 us with 4 iterations to a split, 24
+    // with 2, 22 with 1).
+    const bool by_value = m.data && p.R < kManyRows;
+    const int64_t least_tiles = by_value ? 1 : prefill_split_tiles();
     int prefill_rows = 0;
     int64_t prefill_split = 1;
     double best = 0.0;
@@ -508,10 +517,12 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
         const int in_wg = kFattnPrefillRows / rows;
         const int64_t units = (p.R + rows - 1) / rows * Hkv * B;
         for (int64_t split = 1; split <= prefill_max_split(); ++split) {
-            if (split > 1 && (units * split > n_cu || cell_tiles < prefill_split_tiles() * in_wg * split ||
+            if (split > 4 && (rows == kFattnPrefillRows || units > kFattnDecodeFlagUnits)) break;
+            if (split > 1 && (units * split > n_cu || cell_tiles < least_tiles * in_wg * split ||
                               prefill_scratch(rows, split, units) > ws_bytes))
                 break;
-            const double c = prefill_cost(rows, split, units, (cell_tiles + split * in_wg - 1) / (split * in_wg), n_cu);
+            const double c = prefill_cost(rows, split, units, (cell_tiles + split * in_wg - 1) / (split * in_wg), n_cu,
+                                           by_value);
             if (!prefill_rows || c < best) {
                 prefill_rows = rows;
                 prefill_split = split;
@@ -524,7 +535,7 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
     const int64_t prefill_units = prefill_tiles * Hkv * B;
     // (an explicit mask: the prefill kernel reads its rows 16 bytes at a time)
     const bool mask_rows16 = !m.data || (aligned16(m.data) && m.nb[1] % 16 == 0 && m.nb[2] % 16 == 0 && m.nb[3] % 16 == 0);
-    const bool prefill_shape = !p.dyn && p.R >= (m.data ? kMaskedPrefillRows : prefill_min_rows()) && prefill_units <= kFattnCounterWords &&
+    const bool prefill_shape = !p.dyn && p.R >= prefill_min_rows() && prefill_units <= kFattnCounterWords &&
                                (uint64_t) p.R * (uint64_t) p.G < (1ull << 32) && prefill_tiles * B <= 65535 &&
                                (uint64_t) (n_kv + 64) * k.nb[1] + 256 <= (uint64_t) UINT32_MAX &&
                                (uint64_t) (n_kv + 64) * v.nb[1] + 256 <= (uint64_t) UINT32_MAX && mask_rows16 &&
@@ -532,7 +543,7 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
                                (p.softcap != 0.0f || p.scale > 0.0f) && prefer_prefill();
     if (prefill_shape) {
         pl.kernel = kPrefill;
-        if (p.R >= kMaskedPrefillRows) {
+        if (p.R >= kManyRows) {
             pl.scratch_floor = prefill_scratch_floor(p.R, Hkv * B, cell_tiles, n_cu);
         } else {
             Plan sk = pl;

@@ -55,8 +55,10 @@ hipError_t fattn_splitkv_launch(const FattnParams & p, int rows_per_tile, hipStr
 
 // Prefill kernel: row tiles of rows_per_tile = 128 or 64 query rows (64:
 // two cell splits within the workgroup), n_split workgroups per (kv head,
-// row tile, stream) (1..kFattnPrefillMaxSplit; with more than one, merge
-// records of rows_per_tile rows and arrival counters in the workspace);
+// row tile, stream) (1..kFattnPrefillMaxSplit, 128-row tiles 1..4; with more
+// than one, merge records of rows_per_tile rows in the workspace, with
+// arrival counters, or above 4 the split flags of at most
+// kFattnDecodeFlagUnits tiles);
 // needs fattn_prefill_lds_bytes() of LDS. Masking: the length / causal rule
 // and an explicit mask tensor (rows 16-byte aligned), whose rows the kernel
 // scans for their visible extent; a mask that is not a run of zeros then
@@ -64,7 +66,7 @@ hipError_t fattn_splitkv_launch(const FattnParams & p, int rows_per_tile, hipStr
 hipError_t fattn_prefill_launch(const FattnParams & p, int rows_per_tile, hipStream_t stream);
 size_t fattn_prefill_lds_bytes();
 constexpr int kFattnPrefillRows = 128;          // query rows per workgroup (at most)
-constexpr int kFattnPrefillMaxSplit = 4;        // workgroups sharing one row tile
+constexpr int kFattnPrefillMaxSplit = 32;       // workgroups sharing one row tile
 
 // Decode kernel: up to 32 query rows per kv head (17..32 as two row blocks,
 // 8 x 2 only), one kv head per workgroup, `waves` wavefronts each streaming

@@ -18,8 +18,9 @@
 // LDS at the end. RG = 4 (128 rows, one split) halves the L2 -> LDS traffic
 // per MFMA; RG = 2 (64 rows, two splits) gives twice the workgroups for
 // calls with few rows. When even that does not fill the device, n_split
-// workgroups share a row tile and the last to arrive combines their merge
-// records (the split-KV kernel's record / counter scheme).
+// workgroups share a row tile; the last to arrive combines their merge
+// records (the split-KV kernel's record / counter scheme), or with more than
+// kArrivalSplit of them several do, behind the decode kernel's split flags.
 //
 // Per computing wave and tile (f16 MFMA 32x32x16, f32 accumulation):
 //   S^T[64 cells x 32 rows]  = K Q^T     16 MFMA (two 32-cell blocks, 8 k-steps)
@@ -105,6 +106,101 @@ __device__ __forceinline__ int4v uniform_desc(const char * base, const uint32_t 
                  __builtin_amdgcn_readfirstlane((int) bytes), 0x00020000};
 }
 
+// Publishes this workgroup's rows (64-row tiles; staged in LDS: granule j of
+// row r at j ^ (r & 31), the (m, l) pairs in ml_stage) as a record of n_split
+// > kArrivalSplit: O rows, then the pairs (no line holds both), then the
+// split's flag, and merges: min(n_split, rows / 8) of the unit's workgroups
+// wait for every flag and take rows kidx, kidx + K, ... each, the splits in
+// a fixed order (the decode kernel's hand-off and flag words: flag = epoch +
+// 1, merger 0 advances the epoch; bounded polls). One merging workgroup is
+// bound by the records its CU loads, 34 KB a split.
+constexpr int kArrivalSplit = 4;                 // up to so many splits the last to arrive merges
+__device__ __forceinline__ void merge_many(const float * stage, const float2 * ml_stage, char * lds, const FattnParams & p,
+                                           const rsrc_t rec, const int unit, const int sx, const int b, const int kvh,
+                                           const int row0, const int rows_here, const int tid) {
+    constexpr int kThreads = 2 * kWaves * 64;
+    constexpr uint32_t RS = 64 * kRowStride * 4, kPairs0 = 64 * 512;
+    const int lane = tid & 63;
+    unsigned * flags = p.counters + kFattnCounterWords + unit * kFattnDecodeFlagWords;
+    for (int i = tid; i < rows_here * 32; i += kThreads) {
+        const int r = i >> 5, j = i & 31;
+        buf_store16_dev(*(const float4 *) (stage + r * 128 + 4 * (j ^ (r & 31))), rec, (uint32_t) sx * RS + (uint32_t) i * 16);
+    }
+    if (tid < rows_here)
+        buf_store8_dev(ml_stage[tid], rec, (uint32_t) sx * RS + kPairs0 + (uint32_t) tid * 8);
+    unsigned epoch = 0;
+    if (tid < 64) epoch = ld_agent_u32(flags + 32);
+    complete_wave_memops();
+    __syncthreads();
+    if (tid == 0) st_agent_u32(flags + sx, epoch + 1u);
+    const int K = min(p.n_split, (rows_here + 7) / 8);
+    const int kidx = ((p.n_split - 1 - sx - unit % 8) % p.n_split + p.n_split) % p.n_split;
+    if (kidx >= K) return;
+    int * const merge_failed = (int *) lds;
+    if (tid < 64) {
+        int gave_up = 0;
+        for (int tries = 0;; ++tries) {
+            const unsigned f = lane < p.n_split ? ld_agent_u32(flags + lane) : epoch + 1u;
+            if (__all(f == epoch + 1u)) break;
+            if (tries >= kFlagPollLimit) {
+                gave_up = 1;
+                if (lane == 0) atomicCAS(p.err + 2, 0, 1);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        order_after_counter();
+        if (kidx == 0 && lane == 0 && !gave_up) st_agent_u32(flags + 32, epoch + 1u);
+        if (lane == 0) *merge_failed = gave_up;
+    }
+    __syncthreads();
+    const bool failed = *merge_failed != 0;
+    // Rows kidx + K lr. Round of 8 rows: thread (lr, d4, half) loads its 4
+    // dims of 16 of the splits, while threads (lr, split) of the first 256 turn
+    // the pairs into weights e^(m - M), shared through LDS with M.
+    const int n_my = (rows_here - kidx + K - 1) / K;
+    float2 * ml_s = (float2 *) (lds + 1024);                           // [8][kMaxSplit]
+    float * m_row = (float *) (ml_s + 8 * kMaxSplit);
+    constexpr int kHalf = kMaxSplit / 2;
+    for (int base = 0; base < n_my; base += 8) {
+        const int half = tid & 1, d4 = (tid >> 1) & 31, lr = tid >> 6;
+        const int rr = kidx + K * min(base + lr, n_my - 1);
+        const int pr = kidx + K * min(base + tid / kMaxSplit, n_my - 1), psp = tid % kMaxSplit;
+        float2 ml = {-AL_INF, 0.0f};
+        if (tid < 8 * kMaxSplit && psp < p.n_split)
+            ml = buf_load8_dev(rec, (uint32_t) psp * RS + kPairs0 + (uint32_t) pr * 8);
+        float4 ov[kHalf];
+#pragma unroll
+        for (int j = 0; j < kHalf; ++j)
+            ov[j] = buf_load16_dev(rec, (uint32_t) min(half * kHalf + j, p.n_split - 1) * RS + (uint32_t) (rr * 512 + d4 * 16));
+        if (base > 0) __syncthreads();                                 // the last round's weights are read
+        if (tid < 8 * kMaxSplit) {
+            const float M = max32(ml.x);
+            ml_s[tid] = float2{exp_fast(ml.x - (M == -AL_INF ? 0.0f : M)), ml.y};
+            if (psp == 0) m_row[tid / kMaxSplit] = M;
+        }
+        __syncthreads();
+        float L = 0.0f;
+        float4 acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < kHalf; ++j) {
+            const float2 w = ml_s[lr * kMaxSplit + half * kHalf + j];
+            L += w.x * w.y;
+            acc.x += w.x * ov[j].x; acc.y += w.x * ov[j].y; acc.z += w.x * ov[j].z; acc.w += w.x * ov[j].w;
+        }
+        L += __shfl_xor(L, 1);
+        acc.x += __shfl_xor(acc.x, 1); acc.y += __shfl_xor(acc.y, 1);
+        acc.z += __shfl_xor(acc.z, 1); acc.w += __shfl_xor(acc.w, 1);
+        if (half == 0 && base + lr < n_my) {
+            const int t = div_g(row0 + rr, p.G, p.g_magic);
+            const int hq = kvh * p.G + row0 + rr - t * p.G;
+            float * out = (float *) (p.dst + ((int64_t) (b * p.T + t) * p.Hq + hq) * p.dst_nb1);
+            const float nan = __builtin_nanf("");
+            *(float4 *) (out + 4 * d4) = failed ? float4{nan, nan, nan, nan} : finalize4(acc, m_row[lr], L, p.sinks, hq);
+        }
+    }
+}
+
 template <int RG, bool SOFTCAP, bool MASK>
 __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const FattnParams p) {
     using S = Shape<RG>;
@@ -130,8 +226,13 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     // (XCD affinity: with Hkv = 8 each head's K/V stays in one XCD's L2),
     // row tiles longest first with a causal mask. No integer division on
     // the way to the first loads except for several streams.
-    const int kvh = blockIdx.x;
-    const int sx = blockIdx.y;                   // workgroup split of the row tile
+    // Many workgroup splits (kArrivalSplit < n_split): split fastest instead,
+    // so that the splits a merging workgroup waits for are dispatched ahead
+    // of any later row tile's, as in the decode kernel; the row tiles of a
+    // (split, head), which read the same cells, still meet on one XCD.
+    const bool many = S::SP == 2 && p.n_split > kArrivalSplit;
+    const int kvh = many ? blockIdx.y : blockIdx.x;
+    const int sx = many ? blockIdx.x : blockIdx.y;   // workgroup split of the row tile
     const int z = blockIdx.z;
     const int zt = p.B == 1 ? z : __builtin_amdgcn_readfirstlane(z % p.n_row_tiles);
     const int b = p.B == 1 ? 0 : __builtin_amdgcn_readfirstlane(z / p.n_row_tiles);
@@ -142,14 +243,16 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     auto tok_of = [&](const int r) { return p.G == 1 ? r : (int) __umulhi((uint32_t) r, p.g_magic); };
 
     // An explicit mask (f16 rows of n_kv cells, 16-byte aligned) is read
-    // here first: every mask row that the tile's rows use (one per token
-    // when the mask is shared by the heads, else one per row) is scanned by
-    // one wavefront, 16 bytes per lane and load, for its last cell that is
-    // not -inf (the row's visible extent) and for whether it is a run of
-    // zeros followed by -inf. When every row is, the mask is exactly the
-    // extent and the tiles run as with the length rule; otherwise the whole
-    // workgroup adds slope * mask to its scores tile by tile (general mode).
-    // The results sit in a V buffer that no tile uses before the loop.
+    // here first: of every mask row that the tile's rows use (one per token
+    // when the mask is shared by the heads, else one per row) one wavefront
+    // scans the cells of this workgroup's tiles, 16 bytes per lane and load,
+    // for the last (the row's visible extent) and the first that is not -inf
+    // and for whether they are a run of zeros followed by -inf. When every
+    // row is, the mask is exactly the extent here and the tiles run as with
+    // the length rule; otherwise the whole workgroup adds slope * mask to its
+    // scores tile by tile (general mode). Either way it takes only its tiles
+    // from the first to the last cell that some row sees. The results sit in
+    // a V buffer that no tile uses before the loop.
     constexpr bool has_mask = MASK;           // the launch picks MASK = (p.mask != nullptr)
     const int t0 = tok_of(row0);
     const int n_units = !has_mask ? 0 : p.m_ne2 == 1 ? tok_of(row0 + rows_here - 1) - t0 + 1 : rows_here;
@@ -160,62 +263,95 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         return p.mask + (int64_t) tok * p.m_nb1 + (int64_t) (p.m_ne2 == 1 ? 0 : hq % p.m_ne2) * p.m_nb2 +
                (int64_t) (p.m_ne3 == 1 ? 0 : b % p.m_ne3) * p.m_nb3;
     };
+    // Tiles: the workgroup's cell splits are s_all = sx SP + si of n_all, split
+    // s_all taking the 64-cell tiles j n_all + s_all of the visible range.
+    const int n_all = p.n_split * S::SP;
+    const int s_all = sx * S::SP + si;
     if constexpr (has_mask) {
-        for (int u = wave; u < n_units; u += 2 * kWaves) {
-            const int r_u = p.m_ne2 == 1 ? max(0, (t0 + u) * p.G - row0) : u;   // a tile row of the unit
-            const char * rowp = mask_row(r_u);
-            int last_fin = -1, last0 = -1, first_inf = INT32_MAX, bad = 0;
-            auto classify = [&](const uint32_t hb, const int c) {
-                if (hb != 0xfc00u) last_fin = max(last_fin, c);
-                if ((hb & 0x7fffu) == 0) last0 = max(last0, c);
-                else if (hb == 0xfc00u) first_inf = min(first_inf, c);
-                else bad = 1;
-            };
-            const int n8 = p.n_kv >> 3;
-            for (int j0 = 0; j0 < n8; j0 += 8 * 64) {
-                uint4 w[8];
+        // cells of the workgroup's tiles: runs of SP tiles, n_all tiles apart;
+        // 16-byte piece q of a row is piece q % kRun of run q / kRun
+        constexpr int kRun = S::SP * kTC / 8;
+        const int rule_hi = p.causal_pos0 >= 0 ? (int) min((int64_t) p.kv_hi, p.causal_pos0 + tok_of(row0 + rows_here - 1) + 1)
+                                               : p.kv_hi;
+        const int rule_nt = (max(rule_hi, 0) + kTC - 1) / kTC;
+        const int n_runs = rule_nt > sx * S::SP ? (rule_nt - sx * S::SP + n_all - 1) / n_all : 0;
+        const int n_q = n_runs * kRun;
+        auto piece = [&](const int q) { return ((q / kRun) * n_all + sx * S::SP) * (kTC / 8) + q % kRun; };
+        const int n8 = p.n_kv >> 3;
+        // two rows of the wave at once; per lane and row, as maxima: the last
+        // cell that is not -inf, less the first, the last 0 (past all cells
+        // when some value is neither), less the first -inf
+        for (int u0 = wave; u0 < n_units; u0 += 4 * kWaves) {
+            int us[2] = {u0, min(u0 + 2 * kWaves, n_units - 1)};
+            const char * rowp[2];
+            int m[2][4];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int j = j0 + 64 * q + lane;
-                    w[q] = j < n8 ? *(const uint4 *) (rowp + 16 * (int64_t) j)
-                                  : uint4{0xfc00fc00u, 0xfc00fc00u, 0xfc00fc00u, 0xfc00fc00u};
+            for (int k = 0; k < 2; ++k) {
+                rowp[k] = mask_row(p.m_ne2 == 1 ? max(0, (t0 + us[k]) * p.G - row0) : us[k]);   // a tile row of the unit
+                m[k][0] = m[k][2] = -1;
+                m[k][1] = m[k][3] = -INT32_MAX;
+            }
+            auto classify = [&](int (&mk)[4], const uint32_t hb, const int c) {
+                if (hb != 0xfc00u) {
+                    mk[0] = max(mk[0], c);
+                    mk[1] = max(mk[1], -c);
+                }
+                if ((hb & 0x7fffu) == 0) mk[2] = max(mk[2], c);
+                else if (hb == 0xfc00u) mk[3] = max(mk[3], -c);
+                else mk[2] = INT32_MAX;
+            };
+            for (int q0 = 0; q0 < n_q; q0 += 4 * 64) {
+                uint4 w[2][4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int i = q0 + 64 * q + lane, j = piece(i);
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                        w[k][q] = i < n_q && j < n8 ? *(const uint4 *) (rowp[k] + 16 * (int64_t) j) : uint4{0, 0, 0, 0};
                 }
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int j = j0 + 64 * q + lane;
-                    if (j >= n8) continue;
-                    // 8 cells at once when they are all +-0 or all -inf (the
-                    // two values a causal mask holds), else value by value
-                    const uint32_t x[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
-                    const bool zeros = ((x[0] | x[1] | x[2] | x[3]) & 0x7fff7fffu) == 0u;
-                    const bool infs = x[0] == 0xfc00fc00u && x[1] == 0xfc00fc00u && x[2] == 0xfc00fc00u &&
-                                      x[3] == 0xfc00fc00u;
-                    if (zeros) {
-                        last_fin = max(last_fin, 8 * j + 7);
-                        last0 = max(last0, 8 * j + 7);
-                    } else if (infs) {
-                        first_inf = min(first_inf, 8 * j);
-                    } else {
+                for (int q = 0; q < 4; ++q) {
+                    const int i = q0 + 64 * q + lane, j = piece(i);
+                    if (i >= n_q || j > n8) continue;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            classify(x[e] & 0xffffu, 8 * j + 2 * e);
-                            classify(x[e] >> 16, 8 * j + 2 * e + 1);
+                    for (int k = 0; k < 2; ++k) {
+                        if (j == n8) {                // the row's last cells, fewer than 8
+                            for (int c = 8 * n8; c < p.n_kv; ++c) classify(m[k], ((const uint16_t *) rowp[k])[c], c);
+                            continue;
+                        }
+                        // 8 cells at once when they are all +-0 or all -inf
+                        // (the two values a causal mask holds), else value by
+                        // value
+                        const uint32_t x[4] = {w[k][q].x, w[k][q].y, w[k][q].z, w[k][q].w};
+                        const bool zeros = ((x[0] | x[1] | x[2] | x[3]) & 0x7fff7fffu) == 0u;
+                        const bool infs = x[0] == 0xfc00fc00u && x[1] == 0xfc00fc00u && x[2] == 0xfc00fc00u &&
+                                          x[3] == 0xfc00fc00u;
+                        if (zeros) {
+                            m[k][0] = max(m[k][0], 8 * j + 7);
+                            m[k][1] = max(m[k][1], -8 * j);
+                            m[k][2] = max(m[k][2], 8 * j + 7);
+                        } else if (infs) {
+                            m[k][3] = max(m[k][3], -8 * j);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                classify(m[k], x[e] & 0xffffu, 8 * j + 2 * e);
+                                classify(m[k], x[e] >> 16, 8 * j + 2 * e + 1);
+                            }
                         }
                     }
                 }
             }
-            for (int c = 8 * n8 + lane; c < p.n_kv; c += 64) classify(((const uint16_t *) rowp)[c], c);
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) {
-                last_fin = max(last_fin, __shfl_xor(last_fin, off));
-                last0 = max(last0, __shfl_xor(last0, off));
-                first_inf = min(first_inf, __shfl_xor(first_inf, off));
-                bad |= __shfl_xor(bad, off);
-            }
-            if (lane == 0) {
-                const bool simple = !bad && last0 < first_inf;
-                mtab[2 * u] = simple ? last0 : last_fin;
-                mtab[2 * u + 1] = simple ? 0 : 1;
+            for (int k = 0; k < 2; ++k) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) m[k][i] = wave_max(m[k][i]);
+                if (lane == 0) {
+                    const bool simple = m[k][2] < -m[k][3];
+                    mtab[4 * us[k]] = simple ? m[k][2] : m[k][0];
+                    mtab[4 * us[k] + 1] = simple ? 0 : 1;
+                    mtab[4 * us[k] + 2] = -m[k][1];
+                }
             }
         }
         __syncthreads();                          // (0) the mask table
@@ -224,7 +360,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     // general mode: some row of the tile is not a run of zeros then -inf
     int general = 0;
     if constexpr (has_mask) {
-        for (int u = lane; u < n_units; u += 64) general |= mtab[2 * u + 1];
+        for (int u = lane; u < n_units; u += 64) general |= mtab[4 * u + 1];
         general = __any(general) ? 1 : 0;
     }
 
@@ -240,22 +376,19 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     // one past the last cell any row of the workgroup sees
     const int rr = 32 * rg + lr;
     const bool rvalid = rr < rows_here;
-    int lim, lim_min, hi_wg;
+    int lim, lim_min, hi_wg, lo_wg = 0;
     if constexpr (has_mask) {
         // every wave evaluates all rows of the tile, then reduces
-        auto row_lim = [&](const int r_) { return min(rule_lim(tok_of(row0 + r_)), mtab[2 * unit_of(r_)]); };
+        auto row_lim = [&](const int r_) { return min(rule_lim(tok_of(row0 + r_)), mtab[4 * unit_of(r_)]); };
         lim = rvalid ? row_lim(rr) : INT32_MAX;
-        int lmin = lim, lmax = -1;
+        int lmin = -lim, lmax = -1, lo = -INT32_MAX;
+        for (int u = lane; u < n_units; u += 64) lo = max(lo, -mtab[4 * u + 2]);
 #pragma unroll
         for (int q = 0; q < RG; ++q)
             if (32 * q + lr < rows_here) lmax = max(lmax, q == rg ? lim : row_lim(32 * q + lr));
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            lmin = min(lmin, __shfl_xor(lmin, off));
-            lmax = max(lmax, __shfl_xor(lmax, off));
-        }
-        lim_min = __builtin_amdgcn_readfirstlane(lmin);
-        hi_wg = __builtin_amdgcn_readfirstlane(lmax) + 1;
+        lim_min = __builtin_amdgcn_readfirstlane(-wave_max(lmin));
+        hi_wg = __builtin_amdgcn_readfirstlane(wave_max(lmax)) + 1;
+        lo_wg = __builtin_amdgcn_readfirstlane(-wave_max(lo));
     } else {
         // the rule does not decrease from row to row: the wave's first row
         // has its smallest limit, the tile's last row the largest (scalar
@@ -270,8 +403,9 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     // NI iterations (a split with one tile fewer runs its last iteration on
     // a tile past hi_wg, which every row masks). Tiles from NI on point past
     // the end of the K/V views: they read zeros without memory traffic.
-    const int n_all = p.n_split * S::SP;
-    const int s_all = sx * S::SP + si;
+    // With a mask, hi_wg and lo_wg (the first cell some row sees) are those
+    // within the workgroup's own tiles, whose iterations below j_lo see
+    // nothing and are left out.
     const int NT = (max(hi_wg, 0) + kTC - 1) / kTC;
     // NI = ceil(NT / n_all) and rot ~ rt min(NI, kRotWindow) / n_row_tiles by
     // multiply-high with the plan's reciprocals (0: divisor 1); rot only
@@ -282,15 +416,18 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     // beyond it (us per layer, 512 tokens over 24576 cells: 64 rows a tile 478
     // -> 261, 128 rows 245 -> 221; 256 tokens over 16384 cells 164 -> 94). No
     // stagger at all is 4 % slower at 1536 cells.
-    const int NI = __builtin_amdgcn_readfirstlane(
+    const int NE = __builtin_amdgcn_readfirstlane(
         p.split_magic ? (int) __umulhi((uint32_t) (NT + n_all - 1), p.split_magic) : NT);
+    const int j_lo = !has_mask || lo_wg >= hi_wg ? 0 : __builtin_amdgcn_readfirstlane(
+        p.split_magic ? (int) __umulhi((uint32_t) (lo_wg / kTC), p.split_magic) : lo_wg / kTC);
+    const int NI = NE - j_lo;
     const int rot = __builtin_amdgcn_readfirstlane(
         NI > 0 ? min((int) __umulhi((uint32_t) (rt * min(NI, kRotWindow)), p.tiles_magic), NI - 1) : 0);
     const int n_vis = max(min(hi_wg, p.n_kv), 1);
     auto tile_c0 = [&](const int i) {                     // branch-free: selects only
         int j = i + rot;
         j = j < NI ? j : j - NI;
-        const int c0 = (j * n_all + s_all) * kTC;
+        const int c0 = ((j_lo + j) * n_all + s_all) * kTC;
         return i < NI ? c0 : n_vis;
     };
 
@@ -394,7 +531,10 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         // and the score MFMAs start from -b instead of 0, so p = exp2(t)
         // takes the scores as they are. Otherwise p = exp2(s c - m c).
         constexpr bool FOLD = !SOFTCAP && !GEN;
-        const float cu = FOLD ? 1.0f : cexp;             // state units -> log2 units
+        // The general mode scales the query rows alike: workgroups sharing a row
+        // tile may differ in mode (each looks at its own cells), and rounding
+        // the rows in two ways would shift their scores against each other.
+        const float cu = SOFTCAP ? cexp : 1.0f;          // state units -> log2 units
         const float tau = kTau * kLog2e / cu;            // kTau in state units
         floatx16 negb = {};                               // -b in every register (folded mode)
         // the row's last visible cell less 4 h: cell c0 + 4 h + off is
@@ -404,16 +544,20 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         const int limh = (GEN && !rvalid ? -1 : lim) - 4 * h;
         float thr = -AL_INF;                              // folded mode: rescale when some t exceeds it
         // general mode: this lane's mask row and the factor of its values
-        // (ALiBi slope, arm.cpp:2294, over the scale the scores lack)
+        // (ALiBi slope, arm.cpp:2294, in the scores' units)
         const _Float16 * mrow = nullptr;
         float mslope = 0.0f;
+        uint2 mv[GEN ? 8 : 1];                            // the tile's mask values: cells 8 w + 4 h .. + 3 in mv[w]
+        // cells of the tile (of this half, bit 16 cb + v for register v of
+        // block cb) that some row of the wave sees
+        uint32_t alive = ~0u;
         if constexpr (GEN) {
             mrow = (const _Float16 *) mask_row(rvalid ? rr : 0);
             const uint32_t hq = (uint32_t) (kvh * p.G + (row0 + rr) - tok_of(row0 + rr) * p.G);
             const float slope = p.max_bias > 0.0f ? (hq < p.n_head_log2 ? powf(p.m0, (float) (hq + 1))
                                                                          : powf(p.m1, (float) (2 * (hq - p.n_head_log2) + 1)))
                                                   : 1.0f;
-            mslope = SOFTCAP ? slope : slope / p.scale;
+            mslope = SOFTCAP ? slope : slope * kLog2e;
         }
         // Q^T B operands: row rr (token r / G, head kvh G + r % G), dims
         // 16 ks + 8 h .. + 7, f16 (RNE), loaded straight into registers; the
@@ -445,7 +589,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             if (!kShareQ || si == 0) {
 #pragma unroll
                 for (int ks = 0; ks < 8; ++ks) {
-                    if constexpr (FOLD) {
+                    if constexpr (!SOFTCAP) {
                         qv[2 * ks] *= cexp;
                         qv[2 * ks + 1] *= cexp;
                     }
@@ -511,6 +655,28 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         };
         // some score of the tile above the rescale threshold (lane maximum mx)
         auto outgrows = [&](const float mx) { return FOLD ? mx > thr : mx > m_run + tau; };
+        // general mode: the mask values of the tile at c0 into mv, before the
+        // work that precedes their use (loaded value by value where they
+        // were used, a tile cost 8 load latencies: an iteration took 4 us and
+        // more, 2.4 now)
+        auto load_mask = [&](const int c0) {
+            const int d = limh - c0;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) {
+                mv[w] = uint2{0, 0};
+                if (8 * w > d) continue;                  // past the row's extent
+                const int c = c0 + 4 * h + 8 * w;
+                if (c + 3 < p.m_ne0) {
+                    mv[w] = *(const uint2 *) (mrow + c);
+                } else {                                  // the end of the row
+                    const uint16_t * m16 = (const uint16_t *) (mrow + c);
+                    uint32_t x[3];
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) x[e] = c + e < p.m_ne0 ? m16[e] : 0u;
+                    mv[w] = uint2{x[0] | x[1] << 16, x[2]};
+                }
+            }
+        };
         // fresh scores: softcap, -inf for cells of a tile that some row of
         // the wave does not wholly see, and the reference max moved when the
         // tile outgrows it (a rare, uniform branch; the first visible tile
@@ -531,29 +697,26 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
                     }
             }
             if constexpr (GEN) {
-                // s + slope * mask in the units the scores are kept in (raw
-                // dot products: the mask term divided by the scale); cells
+                // s + slope * mask in the units the scores are kept in; cells
                 // past the row's extent -inf (arm.cpp:2310-2343)
-                // four cells at a time, each group's loads kept in its slot
-                // (a cold path: few registers rather than latency hiding)
-                // (cell c0 + 4 h + off visible when off <= d; the offsets
-                // are immediates of the compares and loads; padding rows of
-                // a ragged last tile load nothing)
+                // (cell c0 + 4 h + off visible when off <= d)
                 const int d = limh - c0;
-                const _Float16 * mt = mrow + c0 + 4 * h;
+                uint32_t seen = 0;                // bit 16 cb + v: the cell of register v is visible
 #pragma unroll
                 for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-                    for (int w4 = 0; w4 < 4; ++w4) {
-                        const int og = 32 * cb + 8 * w4;
-                        float mv[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) mv[e] = og + e <= d ? (float) mt[og + e] : 0.0f;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            sc[cb][4 * w4 + e] = og + e <= d ? sc[cb][4 * w4 + e] + mslope * mv[e] : -AL_INF;
-                        __builtin_amdgcn_sched_barrier(0);
+                    for (int v = 0; v < 16; ++v) {
+                        const int off = 32 * cb + (v & 3) + 8 * (v >> 2);
+                        const uint2 w = mv[4 * cb + (v >> 2)];
+                        const uint32_t hw = (v & 2) ? w.y : w.x;
+                        const float x = mslope * f16_bits_to_float((uint16_t) (v & 1 ? hw >> 16 : hw));
+                        const bool vis = off <= d && x != -AL_INF;
+                        sc[cb][v] = vis ? sc[cb][v] + x : -AL_INF;
+                        seen |= vis ? 1u << (16 * cb + v) : 0u;
                     }
+                // by any row of the wave (the 32 lanes of a half hold the
+                // same cells)
+                alive = or32(seen);
             } else if (c0 + kTC - 1 > lim_min) {
                 // cell c0 + 4 h + off is visible when off <= d: one register
                 // per tile, the offsets are immediates
@@ -608,6 +771,43 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         // of exponentials and of P V products one after the other left the
         // MFMAs of the second idle behind the first's vector work). The
         // products accumulate in the same order as block by block.
+        // General mode, tile by tile: probabilities and P V of tile i, then the
+        // scores of tile i + 1 in the same registers (the fast loop's two
+        // score tiles, with the mask values, spilled). V of cells that no row
+        // of the wave sees counts as zeros (their probability of 0 times
+        // whatever an unused cell holds).
+        auto apply_gen = [&](const int i, const floatx16 (&sc)[2]) {
+            const float mc = m_run == -AL_INF ? 0.0f : m_run * cu;
+            const bool drop = !__all(alive == ~0u);
+            half8 pf[4];
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    pf[kk][e] = (_Float16) __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kk >> 1][8 * (kk & 1) + e], cu, -mc));
+#pragma unroll
+                for (int e = 0; e < 8; e += 2)
+                    l_run = __builtin_amdgcn_fdot2(half2v{pf[kk][e], pf[kk][e + 1]}, half2v{(_Float16) 1.0f, (_Float16) 1.0f}, l_run, false);
+            }
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                half8 v[4];
+#pragma unroll
+                for (int db = 0; db < 4; ++db) v[db] = v_read(vbuf(i), kk, db);
+                if (drop) {
+                    u32x4 m;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t two = alive >> (8 * kk + 2 * e);
+                        m[e] = (two & 1 ? 0xffffu : 0u) | (two & 2 ? 0xffff0000u : 0u);
+                    }
+#pragma unroll
+                    for (int db = 0; db < 4; ++db) v[db] = as_half8(__builtin_bit_cast(u32x4, v[db]) & m);
+                }
+#pragma unroll
+                for (int db = 0; db < 4; ++db) o[db] = mfma32(v[db], pf[kk], o[db]);
+            }
+        };
         float mx;                                 // lane max of S(i + 1), from body(i) (fast mode)
         auto body = [&](const int i, const bool qk, floatx16 (&cur)[2], floatx16 (&nxt)[2]) {
             const float mc = FOLD || m_run == -AL_INF ? 0.0f : m_run * cexp;
@@ -673,17 +873,15 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
                 __builtin_amdgcn_sched_barrier(0);
             }
             // tail: block 3's products and row sums; S(i + 1) prepared and its
-            // lane maxima taken (fast mode; general mode prepares it after the
-            // body) while they run
+            // lane maxima taken while they run
 #pragma unroll
             for (int w = 0; w < 4; ++w)
                 l_run = __builtin_amdgcn_fdot2(half2v{pf[3][2 * w], pf[3][2 * w + 1]}, one2, l_run, false);
 #pragma unroll
             for (int db = 0; db < 4; ++db) o[db] = mfma32(v3[db], pf[3], o[db]);
             __builtin_amdgcn_sched_barrier(0);
-            constexpr bool fold = !GEN;
             float mx0 = -AL_INF, mx1 = -AL_INF;
-            if (fold && qk) {
+            if (qk) {
                 prepare(nxt, tile_c0(i + 1));
                 float m0 = fmaxf(fmaxf(nxt[0][0], nxt[0][1]), nxt[0][2]);
                 float m1 = fmaxf(fmaxf(nxt[1][0], nxt[1][1]), nxt[1][2]);
@@ -700,12 +898,13 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
 
         floatx16 s0[2], s1[2];
         if (NI > 0) {
-            {
+            auto first_scores = [&](const int t) {    // S(t) in s0, its operands read at once
                 half8 kop[2][8];
+                const int kb_ = kbuf(t);
 #pragma unroll
                 for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
-                    for (int ks = 0; ks < 8; ++ks) kop[cb][ks] = k_read(kbuf(0), cb, ks);
+                    for (int ks = 0; ks < 8; ++ks) kop[cb][ks] = k_read(kb_, cb, ks);
 #pragma unroll
                 for (int cb = 0; cb < 2; ++cb) {
                     floatx16 acc = {};
@@ -713,14 +912,25 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
                     for (int ks = 0; ks < 8; ++ks) acc = mfma32(kop[cb][ks], qf[ks], acc);
                     s0[cb] = acc;
                 }
-                finish_scores(s0, tile_c0(0));
+                finish_scores(s0, tile_c0(t));
+            };
+            if constexpr (GEN) load_mask(tile_c0(0));
+            first_scores(0);
+            if constexpr (GEN) {
+                for (int i = 0; i < NI; ++i) {
+                    __syncthreads();                  // (B_i) K(i + 1), V(i) landed; iteration i - 1 done
+                    if (i + 1 < NI) load_mask(tile_c0(i + 1));
+                    apply_gen(i, s0);
+                    if (i + 1 < NI) first_scores(i + 1);
+                }
+                __syncthreads();                      // (3) rings free
+                return;
             }
             // iteration i: S(i) in s0 for even i, s1 for odd i
             auto iteration = [&](const int i, floatx16 (&cur)[2], floatx16 (&nxt)[2]) {
                 __syncthreads();                  // (B_i) K(i + 1), V(i) landed; iteration i - 1 done
                 body(i, true, cur, nxt);
-                if constexpr (GEN) finish_scores(nxt, tile_c0(i + 1));
-                else if (__any(outgrows(mx))) rescale(nxt);
+                if (__any(outgrows(mx))) rescale(nxt);
             };
             int i = 0;
             for (; i + 2 < NI; i += 2) {
@@ -746,12 +956,13 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         if (MASK && general) compute(std::bool_constant<MASK>{});
         else compute(std::false_type{});
     }
-    const float cu_run = !SOFTCAP && !(MASK && general) ? 1.0f : cexp;   // m_run's units -> log2 units
+    const float cu_run = SOFTCAP ? cexp : 1.0f;   // m_run's units -> log2 units
     float m_nat = m_run == -AL_INF ? -AL_INF : m_run * (cu_run / kLog2e);
     float l_row = pair_sum(l_run);
     // The epilogue's lane, row and half read anew: their LDS offsets are
     // computed here, not held in registers across the loop.
     const int lane_e = lane_id_fresh();
+    const int tid = wave * 64 + lane_e;
     const int he = lane_e >> 5;
     const int rre = 32 * rg + (lane_e & 31);
 
@@ -773,7 +984,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             if (he == 0) *(float2 *) (rec + 128) = float2{m_nat, l_row};
         }
         __syncthreads();
-        for (int item = threadIdx.x; item < rows_here * 32; item += 2 * kWaves * 64) {
+        for (int item = tid; item < rows_here * 32; item += 2 * kWaves * 64) {
             const int r = item >> 5, g = item & 31;
             const float * r0 = (const float *) lds + r * kRowStride;
             const float * r1 = (const float *) lds + (ROWS + r) * kRowStride;
@@ -851,7 +1062,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
                 }
         }
         __syncthreads();
-        for (int item = threadIdx.x; item < rows_here * 32; item += 2 * kWaves * 64) {
+        for (int item = tid; item < rows_here * 32; item += 2 * kWaves * 64) {
             const int r = item >> 5, g = item & 31;
             const int rg_ = row0 + r;
             const int tk = tok_of(rg_), hq = kvh * p.G + rg_ - tk * p.G;
@@ -889,35 +1100,42 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             if (he == 0) ml_stage[rre] = float2{m_nat, l_row};
         }
         __syncthreads();
-        for (int i = threadIdx.x; i < rows_here * kGran; i += 2 * kWaves * 64) {
+        for (int i = tid; i < rows_here * kGran; i += 2 * kWaves * 64) {
+            if (many) break;
             const int r = i / kGran, j = i - r * kGran;
             const float2 ml = ml_stage[r];
             const float4 v = j < 32 ? *(const float4 *) (stage + r * 128 + 4 * (j ^ (r & 31))) : float4{ml.x, ml.y, 0.0f, 0.0f};
             buf_store16_dev(v, rec, (uint32_t) sx * RS + (uint32_t) i * 16);
+        }
+        if constexpr (S::SP == 2) {
+            if (many) {
+                merge_many(stage, ml_stage, lds, p, rec, unit, sx, b, kvh, row0, rows_here, tid);
+                return;
+            }
         }
     }
     complete_wave_memops();
     __syncthreads();
     unsigned * cnt = p.counters + unit;
     int * s_last = (int *) (lds + kLds - 16);                       // past the staged rows
-    if (threadIdx.x == 0) *s_last = (add_agent(cnt, 1u) == (unsigned) (p.n_split - 1));
+    if (tid == 0) *s_last = (add_agent(cnt, 1u) == (unsigned) (p.n_split - 1));
     __syncthreads();
     if (!*s_last) return;
     order_after_counter();
-    if (threadIdx.x == 0) st_agent_u32(cnt, 0u);                     // ready for the next call in stream order
+    if (tid == 0) st_agent_u32(cnt, 0u);                     // ready for the next call in stream order
     // Thread t takes (row, 4 dims) items t, t + 512, ..., kBatch at a time,
     // with every record's loads of the batch in flight at once (no loads for
     // splits past n_split).
     constexpr int kBatch = 4;
-    for (int base = threadIdx.x; base < rows_here * 32; base += kBatch * 2 * kWaves * 64) {
-        float2 ml[kBatch][kMaxPrefillSplit];
-        float4 ov[kBatch][kMaxPrefillSplit];
+    for (int base = tid; base < rows_here * 32; base += kBatch * 2 * kWaves * 64) {
+        float2 ml[kBatch][kArrivalSplit];
+        float4 ov[kBatch][kArrivalSplit];
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
             const int item = min(base + k * 2 * kWaves * 64, rows_here * 32 - 1);
             const int r = item >> 5, d4 = item & 31;
 #pragma unroll
-            for (int s2 = 0; s2 < kMaxPrefillSplit; ++s2) {
+            for (int s2 = 0; s2 < kArrivalSplit; ++s2) {
                 ml[k][s2] = float2{-AL_INF, 0.0f};
                 ov[k][s2] = float4{0, 0, 0, 0};
                 if (s2 < p.n_split) {
@@ -934,12 +1152,12 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             const int r = item >> 5, d4 = item & 31;
             float M = ml[k][0].x;
 #pragma unroll
-            for (int s2 = 1; s2 < kMaxPrefillSplit; ++s2) M = fmaxf(M, ml[k][s2].x);
+            for (int s2 = 1; s2 < kArrivalSplit; ++s2) M = fmaxf(M, ml[k][s2].x);
             const float Mu = M == -AL_INF ? 0.0f : M;
             float L = 0.0f;
             float4 acc = {0, 0, 0, 0};
 #pragma unroll
-            for (int s2 = 0; s2 < kMaxPrefillSplit; ++s2) {
+            for (int s2 = 0; s2 < kArrivalSplit; ++s2) {
                 const float w = s2 < p.n_split ? exp_fast(ml[k][s2].x - Mu) : 0.0f;
                 L += w * ml[k][s2].y;
                 acc.x += w * ov[k][s2].x; acc.y += w * ov[k][s2].y; acc.z += w * ov[k][s2].z; acc.w += w * ov[k][s2].w;
@@ -970,9 +1188,12 @@ static void launch_rg(const FattnParams & p, const dim3 grid, hipStream_t stream
 }
 
 hipError_t fattn_prefill_launch(const FattnParams & p, int rows_per_tile, hipStream_t stream) {
-    if (p.n_split < 1 || p.n_split > kMaxPrefillSplit || (rows_per_tile != 64 && rows_per_tile != 128))
+    if (p.n_split < 1 || (rows_per_tile != 64 && rows_per_tile != 128) ||
+        p.n_split > (rows_per_tile == 64 ? kMaxSplit : kArrivalSplit))
         return hipErrorInvalidValue;
-    const dim3 grid((unsigned) p.Hkv, (unsigned) p.n_split, (unsigned) ((int64_t) p.n_row_tiles * p.B));
+    const bool many = p.n_split > kArrivalSplit;                       // split fastest
+    const dim3 grid((unsigned) (many ? p.n_split : p.Hkv), (unsigned) (many ? p.Hkv : p.n_split),
+                    (unsigned) ((int64_t) p.n_row_tiles * p.B));
     if (rows_per_tile == 128) launch_rg<4>(p, grid, stream);
     else launch_rg<2>(p, grid, stream);
     return hipGetLastError();

@@ -15,7 +15,6 @@ typedef float float2v __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 4;                        // one per SIMD, 32 rows each
 constexpr int kLds = 160 * 1024;                 // the rings of all splits (all of a CU's LDS)
-constexpr int kMaxPrefillSplit = kFattnPrefillMaxSplit;
 constexpr float kLog2e = 1.44269504088896341f;
 
 __device__ __forceinline__ floatx16 mfma32(half8 a, half8 b, floatx16 c) {
@@ -30,6 +29,34 @@ __device__ __forceinline__ float pair_max(float x) {
 __device__ __forceinline__ float pair_sum(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
     return __builtin_bit_cast(float, (int) r[0]) + __builtin_bit_cast(float, (int) r[1]);
+}
+
+// OR of the values of each half of the wave (lanes 0..31, 32..63), in all
+// of its lanes (DPP: quads, their mirrors in 8 and 16 lanes, the half's two
+// rows by a permlane swap).
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u(const uint32_t v) {
+    return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t or32(uint32_t x) {
+    x |= dpp_u<0xB1>(x);
+    x |= dpp_u<0x4E>(x);
+    x |= dpp_u<0x141>(x);
+    x |= dpp_u<0x140>(x);
+    const auto r = __builtin_amdgcn_permlane16_swap((int) x, (int) x, false, false);
+    return (uint32_t) r[0] | (uint32_t) r[1];
+}
+
+// The largest x of the wave, in all of its lanes.
+__device__ __forceinline__ int wave_max(int x) {
+    x = max(x, (int) dpp_u<0xB1>((uint32_t) x));
+    x = max(x, (int) dpp_u<0x4E>((uint32_t) x));
+    x = max(x, (int) dpp_u<0x141>((uint32_t) x));
+    x = max(x, (int) dpp_u<0x140>((uint32_t) x));
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = max((int) r[0], (int) r[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return max((int) q[0], (int) q[1]);
 }
 
 // The lane's index within the wave read anew by v_mbcnt behind an opaque

@@ -44,6 +44,22 @@ __device__ __forceinline__ float2 buf_load8_dev(rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, (int) off, 0, kCoherent));
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+// The largest x of each aligned group of 32 lanes, in all of them: DPP
+// within rows of 16 lanes (lane ^ 1, ^ 2, then the mirrors within 8 and
+// 16), then the group's two rows through a permlane swap.
+__device__ __forceinline__ float max32(float x) {
+    x = fmaxf(x, dpp_f<0xB1>(x));
+    x = fmaxf(x, dpp_f<0x4E>(x));
+    x = fmaxf(x, dpp_f<0x141>(x));
+    x = fmaxf(x, dpp_f<0x140>(x));
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
+    return fmaxf(__builtin_bit_cast(float, (int) r[0]), __builtin_bit_cast(float, (int) r[1]));
+}
+
 template <int RB>
 struct Tile {
     u32x4 k[2][4];                   // [mb][kb] K A-operand chunks

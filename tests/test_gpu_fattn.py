@@ -551,3 +551,59 @@ def test_verify_waves_without_stages_and_one_pass_merge(gpu):
         _case(f"{T} drafts over {n_kv} cells")
         got = run_gpu(q, k, v, scale=SCALE, **kw)
         assert_parity(got, O.attention(q, k, v, scale=SCALE, **kw), what=f"{T} drafts over {n_kv} cells")
+
+
+def _sequence_mask(rng, T, n_kv, rows):
+    """Token t sees a range of cells of its own (token 2 none), as a cache
+    shared by several sequences gives; the cells nobody sees."""
+    m = np.full((1, 1, rows, n_kv), -np.inf, dtype=np.float16)
+    cuts = np.sort(rng.choice(np.arange(1, n_kv), T, replace=False))
+    for t in range(T):
+        if t != 2:
+            m[0, 0, t, (cuts[t - 1] + 3 if t else 0):cuts[t]] = 0
+    return m, np.all(m[0, 0, :T] == -np.inf, axis=0)
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,n_kv", [(16, 32, 8, 4096), (9, 32, 8, 128), (17, 4, 1, 1000), (24, 32, 8, 9000),
+                                           (31, 64, 8, 2048), (40, 8, 8, 520)])
+def test_few_rows_with_masks(gpu, T, Hq, Hkv, n_kv):
+    """33 to 255 query rows per kv head with a mask tensor, a row tile shared
+    by up to 32 workgroups, each looking at the mask of its own cells:
+    sequences of one cache, with not-a-numbers in the cells that nobody sees
+    and a token that sees nothing; a causal prefix, which some workgroups
+    take by its extent while the one with a hole takes it by value; biases
+    with ALiBi; softcap and sinks; and a mask whose rows end inside their
+    last 16 bytes."""
+    from arclight_amd import device, fattn
+    rng = np.random.default_rng(T * 100 + n_kv)
+    q, k, v = O.make_inputs(9000 + T, T=T, Hq=Hq, Hkv=Hkv, n_kv=n_kv)
+    rows = (T + 63) // 64 * 64
+    name = f"{T} tokens of {Hq} heads over {n_kv} cells"
+    m, dead = _sequence_mask(rng, T, n_kv, rows)
+    kd, vd = k.copy(), v.copy()
+    kd[:, dead], vd[:, dead] = np.nan, np.nan
+    _check(f"{name}, sequences", q, kd, vd, m, scale=SCALE)
+    m = O.causal_mask(T, n_kv, n_kv - T - 7, kv_len=n_kv - 3)
+    _check(f"{name}, causal prefix", q, k, v, m, scale=SCALE)
+    q2, k2 = q.copy(), k.copy()
+    q2[..., 0] = rng.choice(np.array([-3.0, 0.0, 2.0, 6.0], dtype=np.float32), size=q.shape[:-1])
+    k2[..., 0] = (0.1 * np.arange(n_kv) % 40).astype(np.float16)[None, :, None]
+    mh = m.copy()
+    mh[0, 0, 3:, n_kv // 2:n_kv // 2 + 2] = -np.inf
+    _check(f"{name}, prefix with a hole, growing scores", q2, k2, v, mh, scale=SCALE)
+    mb = m.copy()
+    mb[0, 0, :T] = np.where(m[0, 0, :T] == 0, rng.uniform(-3, 0, (T, n_kv)), -np.inf).astype(np.float16)
+    _check(f"{name}, biases, ALiBi", q, k, v, mb, scale=SCALE, max_bias=8.0)
+    sinks = rng.standard_normal(Hq).astype(np.float32)
+    _check(f"{name}, biases, softcap + sinks", q, k, v, mb, sinks, scale=SCALE * 3, logit_softcap=4.0)
+    if n_kv == 1000:
+        n = n_kv - 3
+        _case(f"{name}, {n} mask columns")
+        dm = device.DeviceTensor(fattn.upload_mask(mb).buf, abi.AL_TYPE_F16, (1, 1, rows, n),
+                                 (rows * 2 * n_kv, rows * 2 * n_kv, 2 * n_kv, 2), 0, abi.MASK_AXES)
+        out = fattn.flash_attn_ext(fattn.upload_q(q), fattn.upload_kv(np.ascontiguousarray(k[:, :n])),
+                                   fattn.upload_kv(np.ascontiguousarray(v[:, :n])), dm, None, scale=SCALE)
+        device.synchronize()
+        ref = O.attention(q, np.ascontiguousarray(k[:, :n]), np.ascontiguousarray(v[:, :n]),
+                          np.ascontiguousarray(mb[..., :n]), scale=SCALE)
+        assert_parity(out.numpy(np.float32), ref, what="mask row end")
