@@ -601,13 +601,21 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
         // workgroups resident per CU by LDS (160 KiB per CU on gfx950)
         const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, (int64_t) (160 << 10) / (int64_t) decode_lds));
         const int64_t target = (int64_t) n_cu * std::min<int64_t>(per_cu, decode_wgs_per_cu());
-        int64_t n_split = (target + decode_units - 1) / decode_units;
-        // every wave of a split gets at least decode_min_stages() stages
-        n_split = std::min<int64_t>(n_split, std::max<int64_t>(1, nst / (dwaves * decode_min_stages())));
-        n_split = std::max<int64_t>(1, std::min<int64_t>(n_split, decode_max_split()));
-        // split flags: kFattnDecodeFlagWords counter words per unit
-        if (decode_units > kFattnDecodeFlagUnits) n_split = 1;
-        const int64_t cps = (nst + n_split - 1) / n_split;
+        // stages per split, of about n splits a unit
+        auto split_stages = [&](int64_t n) {
+            // every wave of a split gets at least decode_min_stages() stages
+            n = std::min<int64_t>(n, std::max<int64_t>(1, nst / (dwaves * decode_min_stages())));
+            n = std::max<int64_t>(1, std::min<int64_t>(n, decode_max_split()));
+            // split flags: kFattnDecodeFlagWords counter words per unit
+            if (decode_units > kFattnDecodeFlagUnits) n = 1;
+            return (nst + n - 1) / n;
+        };
+        // No more workgroups than fit the device at once, or a few of them run
+        // alone behind the others (masked decode of 12 streams, 96 units: 5
+        // splits 48.6 us a layer with its inputs and projection, 6 splits,
+        // which is 576 workgroups for 512 places, 53.0; 3 streams 23.4 / 27.4,
+        // 20 streams of 64 heads 47.7 / 52.7; 24 streams 68.4 / 67.7).
+        const int64_t cps = split_stages(target / decode_units);
         p.cells_per_split = (int32_t) (cps * 16);
         p.n_split = (int32_t) ((nst + cps - 1) / cps);
         p.interleave = decode_interleave() ? 1 : 0;
@@ -635,6 +643,10 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
             pl.part_offset = kFattnCounterBytes;
             pl.part_bytes = (size_t) decode_units * p.n_split * pl.rows_per_tile * kDecodeRecRow;
         }
+        // the least scratch a caller has to bring: that of the next larger split
+        // (less is refused, not run slower)
+        const int64_t cps_up = split_stages((target + decode_units - 1) / decode_units), up = (nst + cps_up - 1) / cps_up;
+        if (up > 1) pl.scratch_floor = kFattnCounterBytes + (size_t) (decode_units * up * pl.rows_per_tile) * kDecodeRecRow;
         *out = pl;
         return AL_OK;
     }

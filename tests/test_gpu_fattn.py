@@ -564,6 +564,34 @@ def _sequence_mask(rng, T, n_kv, rows):
     return m, np.all(m[0, 0, :T] == -np.inf, axis=0)
 
 
+@pytest.mark.parametrize("B,T,n_kv", [(64, 1, 4608), (33, 1, 200), (12, 3, 2100), (16, 1, 64)])
+def test_decode_leaves_out_stages_nobody_sees(gpu, B, T, n_kv):
+    """Masked decode of several streams over one K/V view: each wave takes
+    the 16-cell stages that some row sees, of up to 144 of its own (three
+    words of results). Runs that begin and end inside a stage, the first, the
+    last or no cell at all, alternate stages, finite biases, and not-a-numbers
+    in the cells that no stream sees; then ALiBi, which takes every stage."""
+    rng = np.random.default_rng(B * 1000 + n_kv)
+    q, k, v = O.make_inputs(88 + B, B=B, T=T, Hq=32, Hkv=8, n_kv=n_kv)
+    k, v = k[:1].copy(), v[:1].copy()
+    m = np.full((B, 1, 64, n_kv), -np.inf, np.float16)
+    for b in range(B):
+        for t in range(T):
+            lo, hi = sorted(rng.integers(0, n_kv, 2))
+            m[b, 0, t, lo:hi + 1] = 0.0
+    m[0, 0, :T] = -np.inf
+    m[1, 0, :T], m[1, 0, :T, 0] = -np.inf, 0.0
+    m[2, 0, :T], m[2, 0, :T, -1] = -np.inf, 0.0
+    m[3, 0, 0] = np.where(np.arange(n_kv) // 16 % 2 == 1, 0.0, -np.inf)
+    m[4, 0, 0] = np.where(np.arange(n_kv) % 1040 == 17, rng.uniform(-2, 0, n_kv), -np.inf)
+    m[..., 16:48] = -np.inf
+    assert_parity(run_gpu(q, k, v, m, scale=SCALE, max_bias=8.0),
+                  O.attention(q, k, v, m, scale=SCALE, max_bias=8.0), what="ALiBi")
+    dead = np.isneginf(m[:, 0, :T]).all(axis=(0, 1))
+    k[:, dead], v[:, dead] = np.nan, np.nan
+    _check(f"{B} streams of {T} tokens over {n_kv} cells", q, k, v, m, scale=SCALE)
+
+
 @pytest.mark.parametrize("T,Hq,Hkv,n_kv", [(16, 32, 8, 4096), (9, 32, 8, 128), (17, 4, 1, 1000), (24, 32, 8, 9000),
                                            (31, 64, 8, 2048), (40, 8, 8, 520)])
 def test_few_rows_with_masks(gpu, T, Hq, Hkv, n_kv):
