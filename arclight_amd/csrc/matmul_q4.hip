@@ -480,10 +480,10 @@ __global__ __launch_bounds__(1024) void gemv_q4_fused_kernel(const char * w, int
         }
         return part;
     };
-    if constexpr (TMAX == 8) {
+    if constexpr (TMAX > 1) {
         float part[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) part[t] = t < T ? dot_t(t) : 0.0f;
+        for (int t = 0; t < 8; ++t) part[t] = t < TMAX && t < T ? dot_t(t) : 0.0f;
         const float tot = wave_sum8_scatter(part, lane);
         const int t = lane >> 3;
         if ((lane & 7) == 0 && t < T) *(float *) (y + (int64_t) t * y_nb1 + (int64_t) row * 4) = tot;
@@ -523,7 +523,12 @@ int launch_fused(const al_tensor * w, const al_tensor * x, const al_tensor * y, 
 
 template <int BPL>
 int launch_fused_t(const al_tensor * w, const al_tensor * x, const al_tensor * y, int N, int K, int T, hipStream_t st) {
-    return T == 1 ? launch_fused<BPL, 1>(w, x, y, N, K, T, st) : launch_fused<BPL, kFusedMaxT>(w, x, y, N, K, T, st);
+    // Every wave loads and quantizes its share of TMAX rows, those past T for
+    // nothing: at 2 to 4 tokens the kernel for 8 took, us per call, K 4096, N
+    // 4096: 5.9 (4 tokens) and 5.2 (2) against 5.3 and 4.3; K 8192, N 5120: 15.9
+    // (4) and 14.5 (3) against 12.7 and 11.5. Same bits.
+    if (T == 1) return launch_fused<BPL, 1>(w, x, y, N, K, T, st);
+    return T <= 4 ? launch_fused<BPL, 4>(w, x, y, N, K, T, st) : launch_fused<BPL, kFusedMaxT>(w, x, y, N, K, T, st);
 }
 
 template <int BL>

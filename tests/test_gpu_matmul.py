@@ -66,6 +66,23 @@ def test_wo_matches_oracle(gpu, K, N, T):
     assert rel < 1e-6, rel
 
 
+@pytest.mark.parametrize("K,N,T", [(4096, 17, 2), (8192, 2561, 3), (12288, 31, 4), (16384, 33, 4), (16384, 33, 5)])
+def test_wo_two_to_five_tokens(gpu, K, N, T):
+    """The kernel for up to four tokens, and five, which take the one for up
+    to eight: ragged row counts at every K."""
+    _case(f"wo K={K} N={N} T={T}")
+    rng = np.random.default_rng(K * 7 + N * 3 + T)
+    w = O.random_q4_0(rng, N, K)
+    x = _activations(rng, T, K)
+    got = _run(w, x)
+    want = O.mul_mat_q4_0(w, x)
+    bound = (K // 32 + 16) * 2 * EPS32 * abs_bound(dequant_q4_0(w), dequant_q8_0(O.quantize_q8_0(x)))
+    err = np.abs(got.astype(np.float64) - want)
+    assert np.all(err <= bound), f"worst {err.max():.3e} at {np.unravel_index((err - bound).argmax(), err.shape)}"
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert rel < 1e-6, rel
+
+
 @pytest.mark.parametrize("K,N,T", [(4096, 15, 9), (4096, 17, 16), (8192, 16, 17), (8192, 2561, 33), (12288, 31, 48),
                                    (16384, 33, 63)])
 def test_wo_token_tiles(gpu, K, N, T):
