@@ -256,7 +256,7 @@ int prefill_split_tiles() {
 // tiles at a time) per iteration over its cell tiles, 2.4 when it takes a
 // mask value by value; workgroups past the CUs wait for a round. With more
 // than one to a row tile the last to arrive loads all their records, or,
-// above four, several share that behind the split flags. So 64 rows against
+// above four, a second launch does. So 64 rows against
 // 128 rows in twice the splits changes sides at about 50 iterations (512
 // tokens of 32 heads: 48.1 against 49.9 us at 3584 cells, 89.6 against 87.0 at
 // 8192, 261 against 221 at 24576), and few row tiles over a long cache go to
@@ -517,7 +517,7 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
         const int in_wg = kFattnPrefillRows / rows;
         const int64_t units = (p.R + rows - 1) / rows * Hkv * B;
         for (int64_t split = 1; split <= prefill_max_split(); ++split) {
-            if (split > 4 && (rows == kFattnPrefillRows || units > kFattnDecodeFlagUnits)) break;
+            if (split > 4 && rows == kFattnPrefillRows) break;
             if (split > 1 && (units * split > n_cu || cell_tiles < least_tiles * in_wg * split ||
                               prefill_scratch(rows, split, units) > ws_bytes))
                 break;

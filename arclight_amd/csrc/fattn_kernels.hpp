@@ -57,8 +57,7 @@ hipError_t fattn_splitkv_launch(const FattnParams & p, int rows_per_tile, hipStr
 // two cell splits within the workgroup), n_split workgroups per (kv head,
 // row tile, stream) (1..kFattnPrefillMaxSplit, 128-row tiles 1..4; with more
 // than one, merge records of rows_per_tile rows in the workspace, with
-// arrival counters, or above 4 the split flags of at most
-// kFattnDecodeFlagUnits tiles);
+// arrival counters, or above 4 a second launch that merges them);
 // needs fattn_prefill_lds_bytes() of LDS. Masking: the length / causal rule
 // and an explicit mask tensor (rows 16-byte aligned), whose rows the kernel
 // scans for their visible extent; a mask that is not a run of zeros then

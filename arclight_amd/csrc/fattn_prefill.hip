@@ -20,7 +20,8 @@
 // calls with few rows. When even that does not fill the device, n_split
 // workgroups share a row tile; the last to arrive combines their merge
 // records (the split-KV kernel's record / counter scheme), or with more than
-// kArrivalSplit of them several do, behind the decode kernel's split flags.
+// kArrivalSplit of them a second launch does. No workgroup waits for another,
+// so calls on several streams cannot keep each other from the device.
 //
 // Per computing wave and tile (f16 MFMA 32x32x16, f32 accumulation):
 //   S^T[64 cells x 32 rows]  = K Q^T     16 MFMA (two 32-cell blocks, 8 k-steps)
@@ -61,6 +62,7 @@
 // into the computing waves' registers; the output rows leave through LDS,
 // 16 bytes per lane over whole rows.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "fattn_prefill_common.hpp"
@@ -106,100 +108,9 @@ __device__ __forceinline__ int4v uniform_desc(const char * base, const uint32_t 
                  __builtin_amdgcn_readfirstlane((int) bytes), 0x00020000};
 }
 
-// Publishes this workgroup's rows (64-row tiles; staged in LDS: granule j of
-// row r at j ^ (r & 31), the (m, l) pairs in ml_stage) as a record of n_split
-// > kArrivalSplit: O rows, then the pairs (no line holds both), then the
-// split's flag, and merges: min(n_split, rows / 8) of the unit's workgroups
-// wait for every flag and take rows kidx, kidx + K, ... each, the splits in
-// a fixed order (the decode kernel's hand-off and flag words: flag = epoch +
-// 1, merger 0 advances the epoch; bounded polls). One merging workgroup is
-// bound by the records its CU loads, 34 KB a split.
-constexpr int kArrivalSplit = 4;                 // up to so many splits the last to arrive merges
-__device__ __forceinline__ void merge_many(const float * stage, const float2 * ml_stage, char * lds, const FattnParams & p,
-                                           const rsrc_t rec, const int unit, const int sx, const int b, const int kvh,
-                                           const int row0, const int rows_here, const int tid) {
-    constexpr int kThreads = 2 * kWaves * 64;
-    constexpr uint32_t RS = 64 * kRowStride * 4, kPairs0 = 64 * 512;
-    const int lane = tid & 63;
-    unsigned * flags = p.counters + kFattnCounterWords + unit * kFattnDecodeFlagWords;
-    for (int i = tid; i < rows_here * 32; i += kThreads) {
-        const int r = i >> 5, j = i & 31;
-        buf_store16_dev(*(const float4 *) (stage + r * 128 + 4 * (j ^ (r & 31))), rec, (uint32_t) sx * RS + (uint32_t) i * 16);
-    }
-    if (tid < rows_here)
-        buf_store8_dev(ml_stage[tid], rec, (uint32_t) sx * RS + kPairs0 + (uint32_t) tid * 8);
-    unsigned epoch = 0;
-    if (tid < 64) epoch = ld_agent_u32(flags + 32);
-    complete_wave_memops();
-    __syncthreads();
-    if (tid == 0) st_agent_u32(flags + sx, epoch + 1u);
-    const int K = min(p.n_split, (rows_here + 7) / 8);
-    const int kidx = ((p.n_split - 1 - sx - unit % 8) % p.n_split + p.n_split) % p.n_split;
-    if (kidx >= K) return;
-    int * const merge_failed = (int *) lds;
-    if (tid < 64) {
-        int gave_up = 0;
-        for (int tries = 0;; ++tries) {
-            const unsigned f = lane < p.n_split ? ld_agent_u32(flags + lane) : epoch + 1u;
-            if (__all(f == epoch + 1u)) break;
-            if (tries >= kFlagPollLimit) {
-                gave_up = 1;
-                if (lane == 0) atomicCAS(p.err + 2, 0, 1);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        order_after_counter();
-        if (kidx == 0 && lane == 0 && !gave_up) st_agent_u32(flags + 32, epoch + 1u);
-        if (lane == 0) *merge_failed = gave_up;
-    }
-    __syncthreads();
-    const bool failed = *merge_failed != 0;
-    // Rows kidx + K lr. Round of 8 rows: thread (lr, d4, half) loads its 4
-    // dims of 16 of the splits, while threads (lr, split) of the first 256 turn
-    // the pairs into weights e^(m - M), shared through LDS with M.
-    const int n_my = (rows_here - kidx + K - 1) / K;
-    float2 * ml_s = (float2 *) (lds + 1024);                           // [8][kMaxSplit]
-    float * m_row = (float *) (ml_s + 8 * kMaxSplit);
-    constexpr int kHalf = kMaxSplit / 2;
-    for (int base = 0; base < n_my; base += 8) {
-        const int half = tid & 1, d4 = (tid >> 1) & 31, lr = tid >> 6;
-        const int rr = kidx + K * min(base + lr, n_my - 1);
-        const int pr = kidx + K * min(base + tid / kMaxSplit, n_my - 1), psp = tid % kMaxSplit;
-        float2 ml = {-AL_INF, 0.0f};
-        if (tid < 8 * kMaxSplit && psp < p.n_split)
-            ml = buf_load8_dev(rec, (uint32_t) psp * RS + kPairs0 + (uint32_t) pr * 8);
-        float4 ov[kHalf];
-#pragma unroll
-        for (int j = 0; j < kHalf; ++j)
-            ov[j] = buf_load16_dev(rec, (uint32_t) min(half * kHalf + j, p.n_split - 1) * RS + (uint32_t) (rr * 512 + d4 * 16));
-        if (base > 0) __syncthreads();                                 // the last round's weights are read
-        if (tid < 8 * kMaxSplit) {
-            const float M = max32(ml.x);
-            ml_s[tid] = float2{exp_fast(ml.x - (M == -AL_INF ? 0.0f : M)), ml.y};
-            if (psp == 0) m_row[tid / kMaxSplit] = M;
-        }
-        __syncthreads();
-        float L = 0.0f;
-        float4 acc = {0, 0, 0, 0};
-#pragma unroll
-        for (int j = 0; j < kHalf; ++j) {
-            const float2 w = ml_s[lr * kMaxSplit + half * kHalf + j];
-            L += w.x * w.y;
-            acc.x += w.x * ov[j].x; acc.y += w.x * ov[j].y; acc.z += w.x * ov[j].z; acc.w += w.x * ov[j].w;
-        }
-        L += __shfl_xor(L, 1);
-        acc.x += __shfl_xor(acc.x, 1); acc.y += __shfl_xor(acc.y, 1);
-        acc.z += __shfl_xor(acc.z, 1); acc.w += __shfl_xor(acc.w, 1);
-        if (half == 0 && base + lr < n_my) {
-            const int t = div_g(row0 + rr, p.G, p.g_magic);
-            const int hq = kvh * p.G + row0 + rr - t * p.G;
-            float * out = (float *) (p.dst + ((int64_t) (b * p.T + t) * p.Hq + hq) * p.dst_nb1);
-            const float nan = __builtin_nanf("");
-            *(float4 *) (out + 4 * d4) = failed ? float4{nan, nan, nan, nan} : finalize4(acc, m_row[lr], L, p.sinks, hq);
-        }
-    }
-}
+// Up to so many workgroups of a row tile, the last to arrive merges their
+// records; more leave that to prefill_merge_kernel.
+constexpr int kArrivalSplit = 4;
 
 template <int RG, bool SOFTCAP, bool MASK>
 __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const FattnParams p) {
@@ -226,13 +137,8 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     // (XCD affinity: with Hkv = 8 each head's K/V stays in one XCD's L2),
     // row tiles longest first with a causal mask. No integer division on
     // the way to the first loads except for several streams.
-    // Many workgroup splits (kArrivalSplit < n_split): split fastest instead,
-    // so that the splits a merging workgroup waits for are dispatched ahead
-    // of any later row tile's, as in the decode kernel; the row tiles of a
-    // (split, head), which read the same cells, still meet on one XCD.
-    const bool many = S::SP == 2 && p.n_split > kArrivalSplit;
-    const int kvh = many ? blockIdx.y : blockIdx.x;
-    const int sx = many ? blockIdx.x : blockIdx.y;   // workgroup split of the row tile
+    const int kvh = blockIdx.x;
+    const int sx = blockIdx.y;                   // workgroup split of the row tile
     const int z = blockIdx.z;
     const int zt = p.B == 1 ? z : __builtin_amdgcn_readfirstlane(z % p.n_row_tiles);
     const int b = p.B == 1 ? 0 : __builtin_amdgcn_readfirstlane(z / p.n_row_tiles);
@@ -1075,7 +981,8 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
 
     // Workgroup splits: publish this workgroup's record [unit][sx][row][132]
     // with device-coherent stores; the last workgroup of the row tile to
-    // arrive combines the records of all of them (fixed order) into dst.
+    // arrive, or with more than kArrivalSplit the merge launch, combines the
+    // records of all of them (fixed order) into dst.
     // The record goes out as whole lines: the owners put their rows into LDS
     // (as the finished rows above), then all threads store consecutive
     // 16-byte granules of the record, so every write covers whole lines
@@ -1101,19 +1008,13 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         }
         __syncthreads();
         for (int i = tid; i < rows_here * kGran; i += 2 * kWaves * 64) {
-            if (many) break;
             const int r = i / kGran, j = i - r * kGran;
             const float2 ml = ml_stage[r];
             const float4 v = j < 32 ? *(const float4 *) (stage + r * 128 + 4 * (j ^ (r & 31))) : float4{ml.x, ml.y, 0.0f, 0.0f};
             buf_store16_dev(v, rec, (uint32_t) sx * RS + (uint32_t) i * 16);
         }
-        if constexpr (S::SP == 2) {
-            if (many) {
-                merge_many(stage, ml_stage, lds, p, rec, unit, sx, b, kvh, row0, rows_here, tid);
-                return;
-            }
-        }
     }
+    if (S::SP == 2 && p.n_split > kArrivalSplit) return;              // prefill_merge_kernel merges
     complete_wave_memops();
     __syncthreads();
     unsigned * cnt = p.counters + unit;
@@ -1170,6 +1071,62 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     }
 }
 
+// Rows merged by a workgroup of prefill_merge_kernel, one by each wave.
+constexpr int kMergeRows = 4;
+
+// Combines the records of row tiles (64 rows) shared by more than
+// kArrivalSplit workgroups into dst, in a launch behind theirs: one wavefront
+// per row, lane (half, d4) adding its 4 dims of 16 of the at most 32 splits in
+// order, then the halves. In one launch with the tiles the merge is either
+// the last workgroup's alone, bound by the records that one CU loads (34 KB a
+// split), or that of several that wait for each other's flags, which another
+// stream's workgroups can keep waiting.
+__global__ __launch_bounds__(kMergeRows * 64) void prefill_merge_kernel(const FattnParams p) {
+    __shared__ __attribute__((aligned(16))) float2 w_s[kMergeRows][kMaxSplit];
+    prefetch_params(p);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kvh = blockIdx.y, z = blockIdx.z;
+    const int rt = p.B == 1 ? z : z % p.n_row_tiles, b = p.B == 1 ? 0 : z / p.n_row_tiles;
+    const int r = blockIdx.x * kMergeRows + wave, row = rt * Shape<2>::ROWS + r;
+    if (row >= p.R) return;
+    constexpr uint32_t RS = Shape<2>::ROWS * kRowStride * 4;
+    const int unit = (b * p.Hkv + kvh) * p.n_row_tiles + rt;
+    const rsrc_t rec = make_rsrc(p.part + (int64_t) unit * p.n_split * (RS / 4), RS * (uint32_t) p.n_split);
+    const uint32_t row_off = (uint32_t) (r * kRowStride * 4);
+    // (splits past n_split lie past the records: zeros)
+    const int half = lane >> 5, d4 = lane & 31;
+    float2 ml = buf_load8(rec, (uint32_t) d4 * RS + row_off + 128 * 4);
+    if (d4 >= p.n_split) ml.x = -AL_INF;
+    constexpr int kHalf = kMaxSplit / 2;
+    float4 ov[kHalf];
+#pragma unroll
+    for (int j = 0; j < kHalf; ++j)
+        ov[j] = __builtin_bit_cast(float4, buf_load16(rec, (uint32_t) (half * kHalf + j) * RS + row_off + (uint32_t) (d4 * 16)));
+    static_assert(kMaxSplit == 32, "a row's pairs are the 32 lanes max32 reduces");
+    const float M = max32(ml.x);
+    if (half == 0) w_s[wave][d4] = float2{exp_fast(ml.x - (M == -AL_INF ? 0.0f : M)), ml.y};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float L = 0.0f;
+    float4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < kHalf; ++j) {
+        const float2 w = w_s[wave][half * kHalf + j];
+        L += w.x * w.y;
+        acc.x += w.x * ov[j].x; acc.y += w.x * ov[j].y; acc.z += w.x * ov[j].z; acc.w += w.x * ov[j].w;
+    }
+    L += __shfl_xor(L, 32);
+    acc.x += __shfl_xor(acc.x, 32); acc.y += __shfl_xor(acc.y, 32);
+    acc.z += __shfl_xor(acc.z, 32); acc.w += __shfl_xor(acc.w, 32);
+    if (half == 0) {
+        const int t = div_g(row, p.G, p.g_magic);
+        const int hq = kvh * p.G + row - t * p.G;
+        float * out = (float *) (p.dst + ((int64_t) (b * p.T + t) * p.Hq + hq) * p.dst_nb1);
+        *(float4 *) (out + 4 * d4) = finalize4(acc, M, L, p.sinks, hq);
+    }
+}
+
 }  // namespace
 
 size_t fattn_prefill_lds_bytes() { return (size_t) kLds; }
@@ -1191,10 +1148,15 @@ hipError_t fattn_prefill_launch(const FattnParams & p, int rows_per_tile, hipStr
     if (p.n_split < 1 || (rows_per_tile != 64 && rows_per_tile != 128) ||
         p.n_split > (rows_per_tile == 64 ? kMaxSplit : kArrivalSplit))
         return hipErrorInvalidValue;
-    const bool many = p.n_split > kArrivalSplit;                       // split fastest
-    const dim3 grid((unsigned) (many ? p.n_split : p.Hkv), (unsigned) (many ? p.Hkv : p.n_split),
-                    (unsigned) ((int64_t) p.n_row_tiles * p.B));
+    const unsigned tiles = (unsigned) ((int64_t) p.n_row_tiles * p.B);
+    const dim3 grid((unsigned) p.Hkv, (unsigned) p.n_split, tiles);
     if (rows_per_tile == 128) launch_rg<4>(p, grid, stream);
     else launch_rg<2>(p, grid, stream);
+    if (p.n_split > kArrivalSplit) {
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const unsigned groups = (unsigned) ((std::min(p.R, Shape<2>::ROWS) + kMergeRows - 1) / kMergeRows);
+        hipLaunchKernelGGL(prefill_merge_kernel, dim3(groups, (unsigned) p.Hkv, tiles), dim3(kMergeRows * 64), 0, stream, p);
+    }
     return hipGetLastError();
 }

@@ -40,6 +40,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void buf_store8_dev(float2 v, rsrc_t r, uint32_t off) {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int) off, 0, kCoherent);
 }
+__device__ __forceinline__ float2 buf_load8(rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, (int) off, 0, 0));
+}
 __device__ __forceinline__ float2 buf_load8_dev(rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, (int) off, 0, kCoherent));
 }

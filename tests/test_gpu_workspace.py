@@ -7,6 +7,8 @@
   kernel takes value by value (a hole, biases).
 - Masked many-row calls on two streams, one mask a causal prefix and one
   not, overlap without touching each other's records.
+- Prefill row tiles shared by many workgroups leave the split flags alone
+  and run on two streams at once.
 - A captured masked call replayed first with a non-prefix mask and then with
   a prefix one gives the oracle's result on every replay (nothing a call
   decides about its mask outlives the call).
@@ -191,6 +193,59 @@ def test_split_flags_and_counters_across_calls(gpu):
         flags = words[half:].reshape(-1, 64)[:8]      # the 8 kv heads of stream 0
         assert (flags[:, 32] == epoch).all(), f"{name}: epochs {flags[:, 32]} != {epoch}"
         assert (flags[:, 0] == epoch).all(), f"{name}: split 0 flags {flags[:, 0]} != {epoch}"
+
+
+@pytest.mark.parametrize("T,n_kv,pos0,need_splits", [(16, 8192, 8000, 21), (37, 4096, 4000, 8), (63, 8192, 8129, 8),
+                                                     (48, 1280, 1232, 5)])
+def test_shared_row_tiles_wait_for_nobody(gpu, T, n_kv, pos0, need_splits):
+    """Row tiles of the prefill kernel shared by 5 to 32 workgroups are merged
+    by a launch of their own: the call uses neither the decode kernel's split
+    flags nor their epochs (a waiting workgroup could be kept waiting by
+    another stream's, each filling a CU) and leaves the arrival counters at
+    zero, between decode calls on the same workspace that do use the flags;
+    and calls of such row tiles overlap on two streams."""
+    from arclight_amd import device, fattn
+    region = 256 << 10
+    half = region // 8
+    ws = device.DeviceBuffer(region + (20 << 20))
+    ws.zero()
+    device.synchronize()
+    q, k, v = O.make_inputs(300 + T, T=T, Hq=32, Hkv=8, n_kv=n_kv)
+    kw = dict(kv_len=pos0 + T, causal_pos0=pos0)
+    ref = O.attention(q, k, v, scale=SCALE, **kw)
+    dq, dk, dv = fattn.upload_q(q), fattn.upload_kv(k), fattn.upload_kv(v)
+    need = fattn.workspace_bytes(dq, dk, dv, None, None, _dst(q), scale=SCALE, **kw)
+    tiles = (T * 4 + 63) // 64
+    assert need >= region + tiles * 8 * need_splits * 64 * 528, "row tiles shared by fewer workgroups than meant"
+    q1, k1, v1 = O.make_inputs(31, T=1, Hq=32, Hkv=8, n_kv=4096)
+    ref1 = O.attention(q1, k1, v1, scale=SCALE, kv_len=4000)
+    for rnd in range(2):
+        _case(f"decode, then {T} tokens over {n_kv} cells, round {rnd}")
+        assert_parity(run_gpu(q1, k1, v1, scale=SCALE, workspace=ws, kv_len=4000), ref1, what="decode")
+        before = ws.download(np.empty(region // 4, np.uint32)).copy()
+        assert_parity(run_gpu(q, k, v, scale=SCALE, workspace=ws, **kw), ref, what=f"{T} tokens")
+        after = ws.download(np.empty(region // 4, np.uint32))
+        assert not after[:half].any(), "arrival counters left"
+        assert np.array_equal(before[half:], after[half:]), "split flags or epochs touched"
+    _case(f"{T} tokens over {n_kv} cells on two streams")
+    sa, sb = device.Stream(), device.Stream()
+    try:
+        outs = [_dst(q) for _ in range(8)]
+        for s in (sa, sb):                           # each stream's workspace
+            fattn.flash_attn_ext(dq, dk, dv, scale=SCALE, dst=outs[0], stream=s, **kw)
+        device.synchronize()
+        for i, out in enumerate(outs):
+            fattn.flash_attn_ext(dq, dk, dv, scale=SCALE, dst=out, stream=(sa, sb)[i % 2], **kw)
+        device.synchronize()
+        fattn.device_errors()
+        first = outs[0].numpy(np.float32)
+        assert_parity(first, ref, what="two streams, call 0")
+        for i, out in enumerate(outs[1:], 1):
+            assert np.array_equal(out.numpy(np.float32), first), f"two streams, call {i}"
+    finally:
+        device.synchronize()
+        sa.destroy()
+        sb.destroy()
 
 
 def test_release_stream_workspace(gpu):
