@@ -533,6 +533,16 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
     const int in_wg_split = kFattnPrefillRows / prefill_rows;
     const int64_t prefill_tiles = (p.R + prefill_rows - 1) / prefill_rows;
     const int64_t prefill_units = prefill_tiles * Hkv * B;
+    // Without softcap the prefill kernel takes scale log2(e) into the query
+    // rows before it rounds them to f16. Above 1 a finite row may overflow
+    // there, far below 1 its small values lose bits to f16's denormals (the
+    // error of a score is at most 1 / (scale log2(e)) times that of a row
+    // rounded as it is). Fewer than kManyRows rows then take the split-KV
+    // kernel, and a mask that is no prefix is added to scores of unscaled rows,
+    // which needs one mode for all workgroups of a row tile, so that each
+    // scans the mask rows whole. Qwen3's scale, 1 / sqrt(128), is inside.
+    const float q_factor = p.scale * 1.44269504f;
+    const bool q_folds = p.softcap != 0.0f || (q_factor <= 1.0f && q_factor >= 1.0f / 32.0f);
     // (an explicit mask: the prefill kernel reads its rows 16 bytes at a time)
     const bool mask_rows16 = !m.data || (aligned16(m.data) && m.nb[1] % 16 == 0 && m.nb[2] % 16 == 0 && m.nb[3] % 16 == 0);
     const bool prefill_shape = !p.dyn && p.R >= prefill_min_rows() && prefill_units <= kFattnCounterWords &&
@@ -540,9 +550,10 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
                                (uint64_t) (n_kv + 64) * k.nb[1] + 256 <= (uint64_t) UINT32_MAX &&
                                (uint64_t) (n_kv + 64) * v.nb[1] + 256 <= (uint64_t) UINT32_MAX && mask_rows16 &&
                                lds_per_block >= (int64_t) fattn_prefill_lds_bytes() && q_slice < INT32_MAX &&
-                               (p.softcap != 0.0f || p.scale > 0.0f) && prefer_prefill();
+                               (p.softcap != 0.0f || p.scale > 0.0f) && (p.R >= kManyRows || q_folds) && prefer_prefill();
     if (prefill_shape) {
         pl.kernel = kPrefill;
+        p.mask_whole = m.data && !q_folds;
         if (p.R >= kManyRows) {
             pl.scratch_floor = prefill_scratch_floor(p.R, Hkv * B, cell_tiles, n_cu);
         } else {

@@ -112,7 +112,9 @@ __device__ __forceinline__ int4v uniform_desc(const char * base, const uint32_t 
 // records; more leave that to prefill_merge_kernel.
 constexpr int kArrivalSplit = 4;
 
-template <int RG, bool SOFTCAP, bool MASK>
+// WHOLE (with MASK, without SOFTCAP): p.mask_whole, one mode for all
+// workgroups of a row tile, whose general mode keeps the query rows unscaled.
+template <int RG, bool SOFTCAP, bool MASK, bool WHOLE>
 __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const FattnParams p) {
     using S = Shape<RG>;
     constexpr int ROWS = S::ROWS, NK = S::NK, NV = S::NV, PER = S::PER;
@@ -174,15 +176,17 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     const int n_all = p.n_split * S::SP;
     const int s_all = sx * S::SP + si;
     if constexpr (has_mask) {
-        // cells of the workgroup's tiles: runs of SP tiles, n_all tiles apart;
-        // 16-byte piece q of a row is piece q % kRun of run q / kRun
+        // cells of the workgroup's tiles: runs of SP tiles, n_all tiles apart
+        // (WHOLE: all tiles); 16-byte piece q of a row is piece q %
+        // kRun of run q / kRun
         constexpr int kRun = S::SP * kTC / 8;
+        const int first = WHOLE ? 0 : sx * S::SP, step = WHOLE ? S::SP : n_all;
         const int rule_hi = p.causal_pos0 >= 0 ? (int) min((int64_t) p.kv_hi, p.causal_pos0 + tok_of(row0 + rows_here - 1) + 1)
                                                : p.kv_hi;
         const int rule_nt = (max(rule_hi, 0) + kTC - 1) / kTC;
-        const int n_runs = rule_nt > sx * S::SP ? (rule_nt - sx * S::SP + n_all - 1) / n_all : 0;
+        const int n_runs = rule_nt > first ? (rule_nt - first + step - 1) / step : 0;
         const int n_q = n_runs * kRun;
-        auto piece = [&](const int q) { return ((q / kRun) * n_all + sx * S::SP) * (kTC / 8) + q % kRun; };
+        auto piece = [&](const int q) { return ((q / kRun) * step + first) * (kTC / 8) + q % kRun; };
         const int n8 = p.n_kv >> 3;
         // two rows of the wave at once; per lane and row, as maxima: the last
         // cell that is not -inf, less the first, the last 0 (past all cells
@@ -423,6 +427,10 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
 
     // ---- computing waves ----
     const float cexp = SOFTCAP ? kLog2e : p.scale * kLog2e;
+    // Query rows scaled by cexp before their rounding: the scores come out in
+    // log2 units. Always without softcap in the fast mode; in the general
+    // mode unless WHOLE (below).
+    const float cu = SOFTCAP || (WHOLE && general) ? cexp : 1.0f;   // state units -> log2 units
     floatx16 o[4];
     // m_run in state units: log2 units (s c) in folded mode, else the units
     // of the scores the loop keeps (s, or the softcapped s')
@@ -440,8 +448,10 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         // The general mode scales the query rows alike: workgroups sharing a row
         // tile may differ in mode (each looks at its own cells), and rounding
         // the rows in two ways would shift their scores against each other.
-        const float cu = SOFTCAP ? cexp : 1.0f;          // state units -> log2 units
-        const float tau = kTau * kLog2e / cu;            // kTau in state units
+        // Where scaled rows could leave f16's range (WHOLE) all of a tile's
+        // workgroups look at all cells and so take one mode, and the general
+        // one keeps the rows as they are.
+        const float tau = kTau * kLog2e / (FOLD ? 1.0f : cu);   // kTau in state units
         floatx16 negb = {};                               // -b in every register (folded mode)
         // the row's last visible cell less 4 h: cell c0 + 4 h + off is
         // visible when off <= limh - c0 (padding rows of a ragged last tile:
@@ -463,7 +473,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             const float slope = p.max_bias > 0.0f ? (hq < p.n_head_log2 ? powf(p.m0, (float) (hq + 1))
                                                                          : powf(p.m1, (float) (2 * (hq - p.n_head_log2) + 1)))
                                                   : 1.0f;
-            mslope = SOFTCAP ? slope : slope * kLog2e;
+            mslope = SOFTCAP ? slope : WHOLE ? slope / p.scale : slope * kLog2e;
         }
         // Q^T B operands: row rr (token r / G, head kvh G + r % G), dims
         // 16 ks + 8 h .. + 7, f16 (RNE), loaded straight into registers; the
@@ -495,7 +505,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             if (!kShareQ || si == 0) {
 #pragma unroll
                 for (int ks = 0; ks < 8; ++ks) {
-                    if constexpr (!SOFTCAP) {
+                    if constexpr (!SOFTCAP && !(WHOLE && GEN)) {
                         qv[2 * ks] *= cexp;
                         qv[2 * ks + 1] *= cexp;
                     }
@@ -542,7 +552,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
             const float mt = pair_max(lane_max(sc)) + base;
             const bool g = mt > m_run + tau;
             const float mn = g ? mt : m_run;
-            const float alpha = g ? __builtin_amdgcn_exp2f((m_run - mn) * cu) : 1.0f;   // 0 from -inf
+            const float alpha = g ? __builtin_amdgcn_exp2f((m_run - mn) * (FOLD ? 1.0f : cu)) : 1.0f;   // 0 from -inf
 #pragma unroll
             for (int db = 0; db < 4; ++db) o[db] *= alpha;
             l_run *= alpha;
@@ -862,8 +872,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         if (MASK && general) compute(std::bool_constant<MASK>{});
         else compute(std::false_type{});
     }
-    const float cu_run = SOFTCAP ? cexp : 1.0f;   // m_run's units -> log2 units
-    float m_nat = m_run == -AL_INF ? -AL_INF : m_run * (cu_run / kLog2e);
+    float m_nat = m_run == -AL_INF ? -AL_INF : m_run * (cu / kLog2e);
     float l_row = pair_sum(l_run);
     // The epilogue's lane, row and half read anew: their LDS offsets are
     // computed here, not held in registers across the loop.
@@ -1136,11 +1145,12 @@ static void launch_rg(const FattnParams & p, const dim3 grid, hipStream_t stream
     const dim3 block(2 * kWaves * 64);
     const bool sc = p.softcap != 0.0f, mk = p.mask != nullptr;
     if (sc) {
-        if (mk) hipLaunchKernelGGL((fattn_prefill_kernel<RG, true, true>), grid, block, 0, stream, p);
-        else    hipLaunchKernelGGL((fattn_prefill_kernel<RG, true, false>), grid, block, 0, stream, p);
+        if (mk) hipLaunchKernelGGL((fattn_prefill_kernel<RG, true, true, false>), grid, block, 0, stream, p);
+        else    hipLaunchKernelGGL((fattn_prefill_kernel<RG, true, false, false>), grid, block, 0, stream, p);
     } else {
-        if (mk) hipLaunchKernelGGL((fattn_prefill_kernel<RG, false, true>), grid, block, 0, stream, p);
-        else    hipLaunchKernelGGL((fattn_prefill_kernel<RG, false, false>), grid, block, 0, stream, p);
+        if (mk && p.mask_whole) hipLaunchKernelGGL((fattn_prefill_kernel<RG, false, true, true>), grid, block, 0, stream, p);
+        else if (mk) hipLaunchKernelGGL((fattn_prefill_kernel<RG, false, true, false>), grid, block, 0, stream, p);
+        else    hipLaunchKernelGGL((fattn_prefill_kernel<RG, false, false, false>), grid, block, 0, stream, p);
     }
 }
 

@@ -635,3 +635,35 @@ def test_few_rows_with_masks(gpu, T, Hq, Hkv, n_kv):
         ref = O.attention(q, np.ascontiguousarray(k[:, :n]), np.ascontiguousarray(v[:, :n]),
                           np.ascontiguousarray(mb[..., :n]), scale=SCALE)
         assert_parity(out.numpy(np.float32), ref, what="mask row end")
+
+
+@pytest.mark.parametrize("T,n_kv", [(9, 500), (37, 2048), (64, 2048), (130, 1000)])
+@pytest.mark.parametrize("scale,big", [(1.0, 49152.0), (3.0, 24576.0), (8e-6, 0.0)])
+def test_query_rows_that_scaling_would_move_out_of_f16(gpu, T, n_kv, scale, big):
+    """Queries that f16 holds, with a scale that would take them out of its
+    range if it went into the rows before their rounding: 33 to 255 rows per
+    kv head without a mask, with a prefix mask and with one that has a hole,
+    and from 256 rows on masks with a hole in every row, whose row tiles are
+    shared by several workgroups. Dim 0 carries the large values, exact in
+    f16, against K values that keep the scores within the softmax's reach;
+    with the small scale every K value is large, and scaled rows would keep
+    some 7 bits."""
+    q, k, v = O.make_inputs(61 + T, T=T, Hq=32, Hkv=8, n_kv=n_kv)
+    rng = np.random.default_rng(T)
+    if big:
+        q /= 8 * scale
+        q[..., 0] = big * rng.choice([-1.0, 1.0], q.shape[:-1])
+        k[..., 0] = (3.0 / (big * scale) * rng.uniform(-1, 1, k.shape[:-1])).astype(np.float16)
+    else:
+        k *= np.float16(1e4)
+    name = f"{T} tokens over {n_kv} cells, scale {scale}, |q| to {big}"
+    few = T * 4 < 256
+    if few:
+        _check(f"{name}, causal", q, k, v, scale=scale, kv_len=n_kv, causal_pos0=n_kv - T)
+    m = O.causal_mask(T, n_kv, n_kv - T, kv_len=n_kv)
+    if few:
+        _check(f"{name}, prefix mask", q, k, v, m, scale=scale)
+    m[..., 70] = -np.inf
+    _check(f"{name}, mask with a hole", q, k, v, m, scale=scale)
+    m[..., 90:400] = np.where(m[..., 90:400] == 0, np.float16(-1.25), m[..., 90:400])
+    _check(f"{name}, biases", q, k, v, m, scale=scale)
