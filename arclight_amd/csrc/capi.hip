@@ -141,8 +141,9 @@ static int library_workspace(size_t bytes, void * stream, void ** ptr) {
             w.ptr = nullptr;
             w.bytes = 0;
         }
-        // room for any prefill call (at most one 128-row record a CU) and any
-        // one-stream decode call, so that those never grow it
+        // room for any prefill call (at most one 128-row record a CU, 17 MB)
+        // and any one-stream decode call, so that those never grow it (a
+        // growth waits for the device and fails inside a capture)
         const size_t sz = std::max(bytes, (size_t) 20 << 20);
         hipError_t e = hipMalloc(&w.ptr, sz);
         if (e != hipSuccess) return al_fail(AL_ERR_HIP, "hipMalloc(workspace %zu bytes): %s", sz, hipGetErrorString(e));
@@ -192,7 +193,8 @@ struct Plan {
     size_t part_offset = 0;         // merge records: workspace offset and bytes (0: none)
     size_t part_bytes = 0;
     size_t scratch_floor = 0;       // a caller's scratch below this is refused
-    size_t workspace_bytes() const { return std::max(part_bytes ? part_offset + part_bytes : 0, scratch_floor); }
+    size_t used_bytes() const { return part_bytes ? part_offset + part_bytes : 0; }
+    size_t workspace_bytes() const { return std::max(used_bytes(), scratch_floor); }
 };
 
 bool aligned16(const void * ptr) { return ((uintptr_t) ptr & 15u) == 0; }
@@ -699,7 +701,10 @@ static int fattn_run(const al_fattn_args * a, void * noalloc_ws, size_t noalloc_
                   pl.p.B != 1 || pl.p.mask))
         return al_fail(AL_ERR_UNSUPPORTED, "fattn_with_inputs: the call does not run on the decode kernel "
                        "(up to 16 rows per kv head, one stream, no mask tensor)");
-    const size_t need = pl.workspace_bytes();
+    // what the plan uses; a caller's workspace has to be what
+    // al_fattn_workspace_bytes told the caller
+    const bool callers = !noalloc_ws && a->workspace;
+    const size_t need = callers ? pl.workspace_bytes() : pl.used_bytes();
     if (need) {
         void * ws = noalloc_ws ? noalloc_ws : a->workspace;
         if (noalloc_ws) {

@@ -187,7 +187,8 @@ int al_fattn_apply_node_hints(al_fattn_args * args, const int32_t * op_params);
  */
 int al_fattn_release_stream(void * stream);
 
-/* Workspace bytes al_fattn_f16 needs for these arguments (0 if none). */
+/* Bytes of a caller's workspace that al_fattn_f16 needs for these arguments
+ * (0 if none); with workspace == NULL the library may make do with less. */
 uint64_t al_fattn_workspace_bytes(const al_fattn_args * args);
 
 /*
@@ -199,10 +200,10 @@ uint64_t al_fattn_workspace_bytes(const al_fattn_args * args);
  * records) is a file-scope
  * device array of
  * AL_FATTN_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends. A
- * call that needs more (al_fattn_workspace_bytes) fails with
- * AL_ERR_WORKSPACE. Every call on one GPU shares that array: calls that
- * overlap on one GPU (two streams, or two host threads) race and may give
- * wrong results; order them on one stream.
+ * call whose kernels use more (never more than al_fattn_workspace_bytes)
+ * fails with AL_ERR_WORKSPACE. Every call on one GPU shares that array:
+ * calls that overlap on one GPU (two streams, or two host threads) race and
+ * may give wrong results; order them on one stream.
  * al_fattn_noalloc_init sets up the current device (finds its copy of the
  * array and clears the counter region, synchronizing the default stream):
  * call it once per device before capturing a graph; otherwise the first

@@ -4,8 +4,9 @@ second with a smaller input, each bit-identical to the allocating entry
 point's result (same plan and kernels) and within the parity bar of oracle
 O2 (max-abs <= 2e-3, rel-L2 <= 1e-3). Covers a multi-split decode (counters
 and merge records in the device array), masked many-row calls (one whose
-mask is a causal prefix, one taken value by value), and a call that needs
-more scratch than the array holds (rejected with AL_ERR_WORKSPACE)."""
+mask is a causal prefix, one taken value by value), a call that needs more
+scratch than the array holds (rejected with AL_ERR_WORKSPACE), and one that
+uses none."""
 import ctypes
 import math
 
@@ -84,3 +85,20 @@ def test_noalloc_rejects_oversized_call(gpu):
     _case(f"oversized call ({need} bytes of scratch)")
     assert lib.al_fattn_f16_noalloc(ctypes.byref(a)) == abi.AL_ERR_WORKSPACE
     assert "device array" in lib.al_last_error().decode()
+
+
+def test_noalloc_takes_a_call_that_uses_no_scratch(gpu):
+    """32 tokens of 31 streams over one K/V view: 128 query rows per kv head
+    in 496 row tiles, each one workgroup's, so nothing is merged and the call
+    needs no scratch, although a caller's workspace for it has to be larger
+    than the device array."""
+    from arclight_amd import _lib, abi, device, fattn
+    lib = _lib.load()
+    q, k, v = O.make_inputs(505, B=31, T=32, Hq=32, Hkv=8, n_kv=512)
+    k, v = np.ascontiguousarray(k[:1]), np.ascontiguousarray(v[:1])
+    dst = device.DeviceTensor.empty(q.shape, np.float32, axes=abi.DST_AXES)
+    a = fattn.fattn_args(fattn.upload_q(q), fattn.upload_kv(k), fattn.upload_kv(v), None, None, dst, scale=SCALE)
+    need = lib.al_fattn_workspace_bytes(ctypes.byref(a))
+    assert need > (32 << 20), need
+    _check("32 tokens of 31 streams", q, k, v)
+
