@@ -45,8 +45,6 @@
 // (all loads in flight, fixed order, so results are bit-reproducible) into
 // dst.
 
-#include <type_traits>
-
 #include "fattn_tile.hpp"
 
 namespace {
@@ -280,47 +278,43 @@ __global__ __launch_bounds__(WS * 64) void fattn_decode_kernel(const FattnParams
     const int my_ns = wave_stages(hi);
 
     // The stages the wave takes: the n_pre issued already, then with the
-    // preloaded mask values (MASK 2) those of which some row sees a cell, else
-    // all. A stage nobody sees adds exact zeros, so leaving it out changes no
-    // bit, but its 8 KiB are not streamed: the padding behind a sequence, the
-    // shorter ones of a batch, other sequences' cells in a shared cache.
-    // Lane l tests stage known + l; the word of the 64 results is scalar, so
-    // finding the next stage costs no memory access, and the first word is
-    // made here, once the wave's own values have landed, beside the wait for
-    // the other waves. With ALiBi every stage is taken (a slope that
+    // preloaded mask values (MASK 2) those from the first to the last of which
+    // some row sees a cell, else all. A stage nobody sees adds exact zeros, so
+    // leaving it out changes no bit, but its 8 KiB are not streamed: the
+    // padding behind a sequence, the shorter ones of a batch, idle sequences
+    // in a shared cache. With ALiBi every stage is taken (a slope that
     // underflows to 0 makes NaN of -inf). 12 streams of 1333 to 4000 cells of
-    // a 4096-cell view, 32 heads: 55.2 us, 39 with the stages nobody sees left
-    // out, 35 with 5 splits instead of 6.
-    [[maybe_unused]] int word = n_pre, known = n_pre, issued = n_pre;   // `live`: stages word .. known - 1
-    [[maybe_unused]] uint64_t live = 0;
-    [[maybe_unused]] auto next_word = [&]() {
-        uint32_t seen = p.max_bias > 0.0f ? 1u : 0u;
-        const char * v = mpre + ws * p.mask_wave_bytes + min(known + lane, my_ns - 1) * 32 * p.mask_rows;
-        for (int d = 0; d < p.mask_rows; ++d) {
-            const u32x4 x = *(const u32x4 *) (v + 32 * d), y = *(const u32x4 *) (v + 32 * d + 16);
+    // a 4096-cell view, 32 heads: 55 us, 39 with the stages nobody sees left
+    // out, 35 with 5 splits instead of 6. Two numbers per wave and one loop:
+    // searching the stages one by one, unseen ones in between left out too,
+    // cost one sequence of 9000 cells 0.2 us of 13.7, and as a second copy of
+    // the loop, in a lambda, the unmasked kernels other code (32K cells 28.6
+    // us instead of 26.5).
+    [[maybe_unused]] int n_take = n_pre, jump = 0;                     // stages 0 .. n_pre - 1, then n_pre + jump on
+    [[maybe_unused]] auto find_seen = [&]() {
+        int first = my_ns, last = n_pre - 1;
+        for (int j0 = n_pre; j0 < my_ns; j0 += 64) {                   // lane l tests stage j0 + l
+            uint32_t seen = p.max_bias > 0.0f ? 1u : 0u;
+            const char * v = mpre + ws * p.mask_wave_bytes + min(j0 + lane, my_ns - 1) * 32 * p.mask_rows;
+            for (int d = 0; d < p.mask_rows; ++d) {
+                const u32x4 x = *(const u32x4 *) (v + 32 * d), y = *(const u32x4 *) (v + 32 * d + 16);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) seen |= (x[i] ^ 0xfc00fc00u) | (y[i] ^ 0xfc00fc00u);
+                for (int i = 0; i < 4; ++i) seen |= (x[i] ^ 0xfc00fc00u) | (y[i] ^ 0xfc00fc00u);
+            }
+            const uint64_t live = __ballot(seen != 0 && j0 + lane < my_ns);
+            if (live == 0) continue;
+            first = min(first, j0 + __builtin_ctzll(live));
+            last = j0 + 63 - __builtin_clzll(live);
         }
-        live = __ballot(seen != 0 && known + lane < my_ns);
-        word = known;
-        known += 64;
+        if (last < n_pre) return;
+        jump = first - n_pre;
+        n_take = last + 1 - jump;
     };
-    // the next stage to issue, -1: none left
-    [[maybe_unused]] auto next_live = [&]() {
-        while (live == 0 && known < my_ns) next_word();
-        if (live == 0) return -1;
-        const int j = word + __builtin_ctzll(live);
-        live &= live - 1;
-        return j;
-    };
-    [[maybe_unused]] int stage_of[NB];                                  // the stage in each ring slot
-#pragma unroll
-    for (int u = 0; u < NB; ++u) stage_of[u] = u;
 
     // own query rows landed (the stages were issued after them), then everyone's
     wait_later<NB - 1, PER>(n_pre);
     if constexpr (MASK == 2) {
-        if (known < my_ns) next_word();
+        find_seen();
     }
     __syncthreads();
 
@@ -473,27 +467,17 @@ __global__ __launch_bounds__(WS * 64) void fattn_decode_kernel(const FattnParams
     const int vcell = 4 * g + (n >> 2);                                 // V cell this lane supplies
     const int vread = 4096 + vcell * 256 + (n & 1) * 8;
 
-    auto take_stages = [&](auto skip, const int count) __attribute__((always_inline)) {
-    constexpr bool SKIP = decltype(skip)::value;                        // stages of next_live(), else all of the first `count`
-    for (int i0 = 0; i0 < (SKIP ? issued : count); i0 += NB) {
+    const int count = MASK == 2 ? n_take : my_ns;
+    for (int j0 = 0; j0 < count; j0 += NB) {
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-            if (i0 + u >= (SKIP ? issued : count)) break;
-            const int j = SKIP ? stage_of[u] : i0 + u;
+            int j = j0 + u;
+            if (j >= count) break;
             // this stage landed (own DMA); slot (u + NB - 1) % NB was read
             // last iteration, so the stage NB - 1 ahead may fill it now
-            if constexpr (SKIP) {
-                wait_stage<NB, PER>(issued - 1 - (i0 + u));
-                const int jn = next_live();
-                if (jn >= 0) {
-                    issue(jn, (u + NB - 1) % NB);
-                    stage_of[(u + NB - 1) % NB] = jn;
-                    ++issued;
-                }
-            } else {
-                wait_stage<NB, PER>(min(NB - 2, count - 1 - j));
-                if (j + NB - 1 < count) issue(j + NB - 1, (u + NB - 1) % NB);
-            }
+            wait_stage<NB, PER>(min(NB - 2, count - 1 - j));
+            if (j + NB - 1 < count) issue(j + NB - 1 + jump, (u + NB - 1) % NB);
+            if (MASK == 2 && j >= n_pre) j += jump;
             mem_barrier();
             const char * st = &lds[ws][u][0];
             const int cs = wbase + wstride * j;
@@ -598,16 +582,6 @@ __global__ __launch_bounds__(WS * 64) void fattn_decode_kernel(const FattnParams
 #pragma unroll
                 for (int mb = 0; mb < 8; ++mb) o[rb][mb] = mfma_16x16x16(vt[mb], pf[rb], o[rb][mb]);
         }
-    }
-    };
-    if constexpr (MASK == 2) {
-        // one sequence: the seen stages come first, and the plain loop, whose
-        // next stage is known without a search, takes them (9000 cells of 64
-        // heads: 303 us a step of 12 layers through the search, 297 this way)
-        if (known >= my_ns && (live & (live + 1)) == 0) take_stages(std::false_type{}, n_pre + __builtin_popcountll(live));
-        else take_stages(std::true_type{}, 0);
-    } else {
-        take_stages(std::false_type{}, my_ns);
     }
     // stages issued ahead and not used (my_ns == 0 at run time) land before
     // the rings are reused (with my_ns > 0 the loop's last wait took them)
