@@ -612,8 +612,10 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
         extent = std::max<int64_t>(extent, 0);
         const int64_t nst = std::max<int64_t>(1, (extent + 15) / 16);   // 16-cell stages
         // workgroups resident per CU by LDS (160 KiB per CU on gfx950)
-        const int64_t per_cu = std::max<int64_t>(1, std::min<int64_t>(4, (int64_t) (160 << 10) / (int64_t) decode_lds));
-        const int64_t target = (int64_t) n_cu * std::min<int64_t>(per_cu, decode_wgs_per_cu());
+        auto places = [&](const size_t lds) {
+            return (int64_t) n_cu * std::max<int64_t>(1, std::min<int64_t>((int64_t) (160 << 10) / (int64_t) lds, decode_wgs_per_cu()));
+        };
+        const int64_t target = places(decode_lds + decode_q_lds);
         // stages per split, of about n splits a unit
         auto split_stages = [&](int64_t n) {
             // every wave of a split gets at least decode_min_stages() stages
@@ -627,7 +629,11 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
         // alone behind the others (masked decode of 12 streams, 96 units: 5
         // splits 48.6 us a layer with its inputs and projection, 6 splits,
         // which is 576 workgroups for 512 places, 53.0; 3 streams 23.4 / 27.4,
-        // 20 streams of 64 heads 47.7 / 52.7; 24 streams 68.4 / 67.7).
+        // 20 streams of 64 heads 47.7 / 52.7; 24 streams 68.4 / 67.7). Without
+        // a mask the stage buffers alone would let three on a CU, with the
+        // query rows two fit (attention alone, splits for three against for
+        // two: 3 streams of 4096 cells 17.7 / 14.9, 12 streams 48.6 / 42.6, 24
+        // of 512 cells 19.6 / 15.7, 16 of 4096 58.5 / 58.1).
         const int64_t cps = split_stages(target / decode_units);
         p.cells_per_split = (int32_t) (cps * 16);
         p.n_split = (int32_t) ((nst + cps - 1) / cps);
@@ -656,9 +662,10 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
             pl.part_offset = kFattnCounterBytes;
             pl.part_bytes = (size_t) decode_units * p.n_split * pl.rows_per_tile * kDecodeRecRow;
         }
-        // the least scratch a caller has to bring: that of the next larger split
-        // (less is refused, not run slower)
-        const int64_t cps_up = split_stages((target + decode_units - 1) / decode_units), up = (nst + cps_up - 1) / cps_up;
+        // the least scratch a caller has to bring (less is refused, not run
+        // slower): that of splits for the places of the stage buffers alone,
+        // rounded up
+        const int64_t cps_up = split_stages((places(decode_lds) + decode_units - 1) / decode_units), up = (nst + cps_up - 1) / cps_up;
         if (up > 1) pl.scratch_floor = kFattnCounterBytes + (size_t) (decode_units * up * pl.rows_per_tile) * kDecodeRecRow;
         *out = pl;
         return AL_OK;

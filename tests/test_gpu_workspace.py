@@ -248,6 +248,31 @@ def test_shared_row_tiles_wait_for_nobody(gpu, T, n_kv, pos0, need_splits):
         sb.destroy()
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("B,n_kv", [(3, 4096), (12, 2048), (24, 512)])
+def test_decode_of_streams_fits_the_device_at_once(gpu, B, n_kv, masked):
+    """A decode call of several streams has no more workgroups than the CUs
+    hold at once: two each, by the LDS of the stage buffers and the query
+    rows. The split flags a call leaves in a fresh workspace tell its splits."""
+    from arclight_amd import device, fattn
+    region = 256 << 10
+    ws = device.DeviceBuffer(region + (16 << 20))
+    ws.zero()
+    device.synchronize()
+    q, k, v = O.make_inputs(700 + B, B=B, T=1, Hq=32, Hkv=8, n_kv=n_kv)
+    k, v = np.ascontiguousarray(k[:1]), np.ascontiguousarray(v[:1])
+    m = O.causal_mask(1, n_kv, n_kv - 5, kv_len=n_kv - 4) if masked else None
+    _case(f"{B} streams of {n_kv} cells, {'a mask' if masked else 'no mask'}")
+    kw = {} if masked else dict(kv_len=n_kv - 4)
+    got = run_gpu(q, k, v, m, scale=SCALE, workspace=ws, **kw)
+    ref = O.attention(q[:2], k, v, scale=SCALE, kv_len=n_kv - 4)
+    assert_parity(got[:2], ref, what=f"{B} streams")
+    flags = ws.download(np.empty(region // 4, np.uint32))[region // 8:].reshape(-1, 64)[:B * 8, :32]
+    splits = (flags != 0).sum(axis=1)
+    assert splits.min() == splits.max() > 1
+    assert splits.sum() <= 2 * device.device_info()["n_cu"], splits[0]
+
+
 def test_release_stream_workspace(gpu):
     """al_fattn_release_stream frees a stream's library workspace: split
     decode calls on the stream before and after the release (which
