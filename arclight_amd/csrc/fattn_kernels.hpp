@@ -42,6 +42,7 @@ struct FattnParams {
     int32_t mask_wave_bytes;        //   LDS bytes per wave (whole 1 KiB DMA blocks)
     int32_t one_pass;               // decode kernel, 2 waves: the waves' states merged in one pass
     int32_t mask_whole;             // prefill kernel: one mode for all workgroups of a row tile, the general one with unscaled query rows
+    float   tau;                    // prefill kernel: growth of a row's maximum that moves its reference (natural units)
     float *    part;                // split-KV merge records: [units][n_split][rows per tile][record stride]
     unsigned * counters;            // [units] in the fixed counter region, zero between calls
     int *      err;                 // device error flags (al_device_errors): [0, 1] set_rows, [2] a merge gave up waiting

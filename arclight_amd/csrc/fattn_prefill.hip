@@ -42,7 +42,7 @@
 // started from -b), with softcap or a general mask p = exp2(s' c - m c)
 // from the scores as they are. Row sums accumulate by v_dot2 of the f16 P
 // with ones, and the reference max moves lazily (only when a tile exceeds
-// it by more than kTau in natural units) on a cold path outside the fast
+// it by more than p.tau in natural units) on a cold path outside the fast
 // loop, so the O accumulators stay in the matrix cores' registers there.
 //
 // Memory path. K and V tiles go HBM/L2 -> LDS by LDS-DMA (buffer_load ...
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         // Where scaled rows could leave f16's range (WHOLE) all of a tile's
         // workgroups look at all cells and so take one mode, and the general
         // one keeps the rows as they are.
-        const float tau = kTau * kLog2e / (FOLD ? 1.0f : cu);   // kTau in state units
+        const float tau = p.tau * kLog2e / (FOLD ? 1.0f : cu);   // p.tau in state units
         floatx16 negb = {};                               // -b in every register (folded mode)
         // the row's last visible cell less 4 h: cell c0 + 4 h + off is
         // visible when off <= limh - c0 (padding rows of a ragged last tile:

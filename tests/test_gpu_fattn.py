@@ -667,3 +667,30 @@ def test_query_rows_that_scaling_would_move_out_of_f16(gpu, T, n_kv, scale, big)
     _check(f"{name}, mask with a hole", q, k, v, m, scale=scale)
     m[..., 90:400] = np.where(m[..., 90:400] == 0, np.float16(-1.25), m[..., 90:400])
     _check(f"{name}, biases", q, k, v, m, scale=scale)
+
+
+def test_few_rows_probabilities_follow_the_maximum(gpu):
+    """63 tokens over 8192 cells (252 query rows per kv head): probabilities
+    are rounded to f16 against the largest score, not against an earlier one
+    that the later exceed by up to 8. Queries, keys and their product with
+    the scale's share of a row are exact in 16 bits, so what is left against
+    64 bits is that rounding: at most what numpy makes of it with one maximum
+    for all of a row's cells (the kernel has one for each wave's share of
+    them), which against the first cells' maximum would be half as much
+    again."""
+    T, n_kv = 63, 8192
+    scale = float(np.float32(0.125) / np.float32(1.44269504))
+    q, k, v = O.make_inputs(404, T=T, Hq=32, Hkv=8, n_kv=n_kv)
+    q = (q * 2).astype(np.float16).astype(np.float32)
+    k = (k * np.float16(1.5)).astype(np.float16)
+    _case(f"{T} tokens over {n_kv} cells against 64 bits")
+    got = run_gpu(q, k, v, scale=scale)
+    off, most = [], []
+    for h in range(0, 32, 4):
+        s = q[0, :, h].astype(np.float64) @ k[0, :, h // 4].astype(np.float64).T * scale
+        p, vh = np.exp(s - s.max(-1, keepdims=True)), v[0, :, h // 4].astype(np.float64)
+        pr = p.astype(np.float16).astype(np.float64)
+        exact = p @ vh / p.sum(-1, keepdims=True)
+        off.append(np.linalg.norm(got[0, :, h] - exact))
+        most.append(np.linalg.norm(pr @ vh / pr.sum(-1, keepdims=True) - exact))
+    assert np.linalg.norm(off) <= np.linalg.norm(most), (np.linalg.norm(off), np.linalg.norm(most))
