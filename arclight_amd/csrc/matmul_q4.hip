@@ -541,7 +541,9 @@ int launch_gemm(const al_tensor * w, const al_tensor * y, int N, int tiles, int 
     return e == hipSuccess ? AL_OK : al_hip_fail(e, "mul_mat_q4_0: launch");
 }
 
-// Per-device scratch for the quantized activations, grown on demand.
+// Per-device scratch for the quantized activations; the first allocation
+// has room for every call (64 tokens of K = 16384: 1.1 MB), so that none
+// grows it, which would fail inside a capture.
 struct Scratch {
     void * p = nullptr;
     size_t bytes = 0;
@@ -564,7 +566,7 @@ int scratch(size_t bytes, void ** out) {
             s.p = nullptr;
             s.bytes = 0;
         }
-        const size_t sz = std::max(bytes, (size_t) 1 << 20);
+        const size_t sz = std::max(bytes, (size_t) 2 << 20);
         e = hipMalloc(&s.p, sz);
         if (e != hipSuccess) return al_hip_fail(e, "mul_mat_q4_0: scratch");
         s.bytes = sz;

@@ -142,6 +142,34 @@ def test_wo_repeated_calls_reuse_scratch(gpu):
     assert np.linalg.norm(got - want) / np.linalg.norm(want) < 1e-6
 
 
+def test_wo_first_call_makes_room_for_all(gpu):
+    """After one call of more than 8 tokens, however small, every other call
+    can be captured: 50 and 64 tokens at the largest K need no larger scratch
+    than the 9 tokens before them (as the process's first such call)."""
+    from arclight_amd import device, matmul
+    rng = np.random.default_rng(5)
+    w = O.random_q4_0(rng, 40, 16384)
+    wm = matmul.Q4_0Matrix(w.view(np.uint8), 16384, 40)
+    _run(w[:, :128].copy(), _activations(rng, 9, 4096))
+    for T in (50, 64):
+        x = _activations(rng, T, 16384)
+        xd, yd = device.DeviceTensor.from_numpy(x), device.DeviceTensor.empty((T, 40), np.float32)
+        st = device.Stream()
+        g = device.Graph(st, lambda: matmul.mul_mat_q4_0(wm, xd, yd, stream=st))
+        eager = _run(w, x)
+        try:
+            for i in range(3):
+                _case(f"wo {T} tokens, replay {i}")
+                yd.buf.zero()
+                device.synchronize()
+                g.launch(st)
+                st.synchronize()
+                assert np.array_equal(yd.numpy(np.float32), eager), f"{T} tokens, replay {i}"
+        finally:
+            g.destroy()
+            st.destroy()
+
+
 @pytest.mark.parametrize("K,N,T,status", [(2048, 64, 1, abi.AL_ERR_UNSUPPORTED), (20480, 64, 1, abi.AL_ERR_UNSUPPORTED),
                                           (4096, 64, 65, abi.AL_ERR_UNSUPPORTED)])
 def test_wo_rejects_unsupported_shapes(gpu, K, N, T, status):
