@@ -694,3 +694,30 @@ def test_few_rows_probabilities_follow_the_maximum(gpu):
         off.append(np.linalg.norm(got[0, :, h] - exact))
         most.append(np.linalg.norm(pr @ vh / pr.sum(-1, keepdims=True) - exact))
     assert np.linalg.norm(off) <= np.linalg.norm(most), (np.linalg.norm(off), np.linalg.norm(most))
+
+
+@pytest.mark.parametrize("T,Hq,n_kv", [(10, 32, 700), (25, 64, 1500), (150, 32, 300)])
+def test_negative_scale(gpu, T, Hq, n_kv):
+    """Scores times a negative scale, without a mask and with one: calls of
+    more than 32 rows per kv head stay on the split-KV kernel (its 64-row
+    tiles), one workgroup to a tile and several."""
+    q, k, v = O.make_inputs(71 + T, T=T, Hq=Hq, Hkv=8, n_kv=n_kv)
+    _check(f"{T} tokens of {Hq} heads, scale < 0, causal", q, k, v, scale=-SCALE, kv_len=n_kv, causal_pos0=n_kv - T)
+    _check(f"{T} tokens of {Hq} heads, scale < 0", q, k, v, scale=-SCALE, kv_len=n_kv - 9)
+    _check(f"{T} tokens of {Hq} heads, scale < 0, mask", q, k, v, O.causal_mask(T, n_kv, n_kv - T), scale=-SCALE)
+
+
+@pytest.mark.parametrize("G", [1, 17])
+def test_more_streams_than_the_decode_kernel_counts(gpu, G):
+    """4097 streams of 8 kv heads, more (stream, head) pairs than arrival
+    counters, without a mask: the split-KV kernel's 16- and 32-row tiles. A
+    sample of streams against the oracle."""
+    B, n_kv = 4097, 40
+    rng = np.random.default_rng(G)
+    q = rng.standard_normal((B, 1, 8 * G, 128), dtype=np.float32)
+    _, k, v = O.make_inputs(72, T=1, Hq=8, Hkv=8, n_kv=n_kv)
+    _case(f"{B} streams of {G} heads to a kv head")
+    got = run_gpu(q, k, v, scale=SCALE, kv_len=n_kv - 3)
+    sel = np.unique(np.concatenate([[0, 1, B - 1], rng.choice(B, 20, replace=False)]))
+    assert_parity(got[sel], O.attention(np.ascontiguousarray(q[sel]), k, v, scale=SCALE, kv_len=n_kv - 3),
+                  what=f"{G} heads to a kv head")
