@@ -222,9 +222,9 @@ int env_int(const char * name, int dflt) {
 // Fewest query rows per kv head that go to the prefill kernel
 // (AL_PREFILL_MIN_ROWS); fewer take the decode kernel. Measured, us per layer
 // with the inputs, split-KV against prefill: 9 tokens of 32 heads over 500
-// cells 31.5 / 12.9, over 8000 43.9 / 17.6, 37 over 3000 66 / 17.9, 63 over 8000
-// 95 / 25; with a mask tensor 37 over 3000
-// 83 / 25, 16 sequences in one cache of 16384 cells 89 / 35.
+// cells 31.5 / 12.9, over 8000 43.9 / 17.6, 37 over 3000 66 / 17.9, 63 over
+// 8000 95 / 25; with a mask tensor 37 over 3000 83 / 25, 16 sequences in one
+// cache of 16384 cells 89 / 35.
 int prefill_min_rows() {
     static int v = env_int("AL_PREFILL_MIN_ROWS", 33);
     return v;
@@ -505,10 +505,13 @@ int make_plan(const al_fattn_args * a, int n_cu, int lds_per_block, uint64_t ws_
     int64_t prefill_extent = p.kv_hi;
     if (p.causal_pos0 >= 0) prefill_extent = std::min<int64_t>(prefill_extent, p.causal_pos0 + T);
     const int64_t cell_tiles = std::max<int64_t>(1, (prefill_extent + 63) / 64);
-    // A mask over few rows is as a rule that of several sequences in one
-    // cache, which the kernel takes value by value, with less work to a split
-    // (9 sequences of up to 200 cells: 30 us with 4 iterations to a split, 24
-    // with 2, 22 with 1).
+    // Which mode a mask will take is not known here: it is in device memory.
+    // Few rows are planned as value by value, as a mask of several sequences
+    // in one cache makes them, with less work to a split (9 sequences of up to
+    // 200 cells: 30 us with 4 iterations to a split, 24 with 2, 22 with 1);
+    // many rows as a prefix, which the ubatches of one prompt have. A wrong
+    // guess costs time only: a prefix mask over few rows gets more splits than
+    // the same call without a mask, a mask with holes over many rows fewer.
     const bool by_value = m.data && p.R < kManyRows;
     const int64_t least_tiles = by_value ? 1 : prefill_split_tiles();
     int prefill_rows = 0;

@@ -285,11 +285,13 @@ __global__ __launch_bounds__(WS * 64) void fattn_decode_kernel(const FattnParams
     // in a shared cache. With ALiBi every stage is taken (a slope that
     // underflows to 0 makes NaN of -inf). 12 streams of 1333 to 4000 cells of
     // a 4096-cell view, 32 heads: 55 us, 39 with the stages nobody sees left
-    // out, 35 with 5 splits instead of 6. Two numbers per wave and one loop:
-    // searching the stages one by one, unseen ones in between left out too,
-    // cost one sequence of 9000 cells 0.2 us of 13.7, and as a second copy of
-    // the loop, in a lambda, the unmasked kernels other code (32K cells 28.6
-    // us instead of 26.5).
+    // out, 35 with 5 splits instead of 6. Where there is nothing to leave out
+    // the search costs 0.1 to 0.6 us (9000 cells of 64 heads 13.7 -> 13.9, 32K
+    // of 32 heads 27.0 -> 27.6). Two numbers per wave and one loop: a search
+    // stage by stage, which leaves out unseen ones in between too, wants a
+    // second copy of the loop, and with the loop in a lambda for that the
+    // unmasked kernels compiled to other code (32K cells 28.6 us instead of
+    // 26.5); in the one loop it took 33.7 us.
     [[maybe_unused]] int n_take = n_pre, jump = 0;                     // stages 0 .. n_pre - 1, then n_pre + jump on
     [[maybe_unused]] auto find_seen = [&]() {
         int first = my_ns, last = n_pre - 1;

@@ -19,10 +19,10 @@
 // nibbles, the weights' offset of 8 folded into one multiply by the block's
 // value sum; lane sums meet in a DPP wave reduction.
 // Longer inputs (up to 64 tokens) take two launches: quantize_q8_kernel
-// (into grow-only library scratch, laid out as MFMA operands) and
-// gemm_q4_kernel, whose integer dot products run on the matrix cores.
-// Either way the 4-bit weights stream once: HBM-bound, 18 bytes per 32
-// weights.
+// (into library scratch, laid out as MFMA operands) and gemm_q4_kernel, whose
+// integer dot products run on the matrix cores. The 4-bit weights, 18 bytes
+// per 32, are read from memory once; with more than 16 tokens every tile of
+// 16 reads them again from the caches.
 
 #include <hip/hip_runtime.h>
 
@@ -152,11 +152,14 @@ __global__ __launch_bounds__(256) void quantize_q8_kernel(const char * __restric
 // each of its 8 waves 1/8 of K. One MFMA 16x16x32 i8 is one block's integer
 // dot products of 16 tokens and 16 rows, exact, as the format needs them;
 // its 4 results per lane then cost a conversion, a product and an FMA each.
-// That vector work and the unpacking (723 instructions per wave at K = 8192)
-// bound the kernel, so a workgroup takes one token tile: more would unpack
-// the weights once for several tiles, but leave CUs idle (K 8192, N 5120, 48
-// tokens: 21.4 us with one tile, 27.9 with three; 64 tokens: 25.7 with one,
-// 27.5 with two, 33.0 with four).
+// Nothing is saturated: at K 8192, N 5120 and 48 tokens the 896 vector
+// instructions of a wave take 11.2 of the launch's 19.4 us, the MFMAs 1.6, the
+// LDS 4.6, the 28 MB from memory 6; the rest is waiting, in two rounds of
+// workgroups (960 for 512 places, two a CU by their 106 registers) that each
+// start with their loads exposed. A workgroup takes one token tile: more
+// would unpack the weights once for several tiles, but leave CUs idle (21.4
+// us with one tile, 27.9 with three; 64 tokens: 25.7 with one, 27.5 with two,
+// 33.0 with four).
 // In a step the workgroup takes 64 blocks of every row, a wave 8: lanes 4 r
 // .. 4 r + 3 load row r's 144 bytes of them (a pair of blocks each), so that
 // a load touches few lines, and a permute brings row r's pair g to lane 16 g
@@ -378,8 +381,7 @@ __device__ __forceinline__ float wave_sum8_scatter(const float (&v)[8], const in
 // rows' weight loads, quantizes all T activation rows into LDS meanwhile
 // (they are small and L2-resident after the first workgroup touches them;
 // each thread issues the loads of all T tokens of its part of a block before
-// using any), then runs the dot products of gemv_q4_kernel from LDS. One
-// wavefront per row; with several tokens the rows' per-lane sums of all of
+// using any), then runs the dot products from LDS. One wavefront per row; with several tokens the rows' per-lane sums of all of
 // them meet in one scattering wave reduction.
 template <int BPL, int TMAX>
 __global__ __launch_bounds__(1024) void gemv_q4_fused_kernel(const char * w, int64_t w_nb1, int N, int K,
@@ -495,6 +497,12 @@ __global__ __launch_bounds__(1024) void gemv_q4_fused_kernel(const char * w, int
     }
 }
 
+// Most tokens of the one-launch kernel. Against the two launches for more
+// tokens (us per call): K 4096, N 4096: 7.0 / 8.2 at 5 tokens, 8.3 / 8.2 at 8;
+// K 8192, N 5120: 13.2 / 15.8 at 4, 17.9 / 15.6 at 5, 21.7 / 15.7 at 8. At K
+// 8192 the line for time alone would be 4; calls of 5 to 8 tokens, as verify
+// steps make them, stay here because this kernel needs no scratch, so that
+// they can be captured into a graph whatever ran before.
 constexpr int kFusedMaxT = 8;
 
 size_t fused_lds_bytes(int64_t K, int64_t T) { return (size_t) (T * K + 8 * T * (K / 32)); }   // <= 160 KiB
