@@ -429,8 +429,10 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
     const float cexp = SOFTCAP ? kLog2e : p.scale * kLog2e;
     // Query rows scaled by cexp before their rounding: the scores come out in
     // log2 units. Always without softcap in the fast mode; in the general
-    // mode unless WHOLE (below).
-    const float cu = SOFTCAP || (WHOLE && general) ? cexp : 1.0f;   // state units -> log2 units
+    // mode unless WHOLE (below). The general mode's scores and maxima are in
+    // natural units: beside a mask value of -65504 the sum's last bit is then
+    // the one the operator's definition has, 1/256.
+    const float cu = SOFTCAP || (MASK && general) ? kLog2e : 1.0f;   // state units -> log2 units
     floatx16 o[4];
     // m_run in state units: log2 units (s c) in folded mode, else the units
     // of the scores the loop keeps (s, or the softcapped s')
@@ -460,9 +462,10 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         const int limh = (GEN && !rvalid ? -1 : lim) - 4 * h;
         float thr = -AL_INF;                              // folded mode: rescale when some t exceeds it
         // general mode: this lane's mask row and the factor of its values
-        // (ALiBi slope, arm.cpp:2294, in the scores' units)
+        // (ALiBi slope, arm.cpp:2294), and the scores' natural units
         const _Float16 * mrow = nullptr;
-        float mslope = 0.0f;
+        float slope = 1.0f;
+        const float snat = SOFTCAP ? 1.0f : WHOLE ? p.scale : kLn2;
         uint2 mv[GEN ? 8 : 1];                            // the tile's mask values: cells 8 w + 4 h .. + 3 in mv[w]
         // cells of the tile (of this half, bit 16 cb + v for register v of
         // block cb) that some row of the wave sees
@@ -470,10 +473,8 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         if constexpr (GEN) {
             mrow = (const _Float16 *) mask_row(rvalid ? rr : 0);
             const uint32_t hq = (uint32_t) (kvh * p.G + (row0 + rr) - tok_of(row0 + rr) * p.G);
-            const float slope = p.max_bias > 0.0f ? (hq < p.n_head_log2 ? powf(p.m0, (float) (hq + 1))
-                                                                         : powf(p.m1, (float) (2 * (hq - p.n_head_log2) + 1)))
-                                                  : 1.0f;
-            mslope = SOFTCAP ? slope : WHOLE ? slope / p.scale : slope * kLog2e;
+            if (p.max_bias > 0.0f)
+                slope = hq < p.n_head_log2 ? powf(p.m0, (float) (hq + 1)) : powf(p.m1, (float) (2 * (hq - p.n_head_log2) + 1));
         }
         // Q^T B operands: row rr (token r / G, head kvh G + r % G), dims
         // 16 ks + 8 h .. + 7, f16 (RNE), loaded straight into registers; the
@@ -613,8 +614,8 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
                     }
             }
             if constexpr (GEN) {
-                // s + slope * mask in the units the scores are kept in; cells
-                // past the row's extent -inf (arm.cpp:2310-2343)
+                // s + slope * mask; cells past the row's extent -inf
+                // (arm.cpp:2310-2343)
                 // (cell c0 + 4 h + off visible when off <= d)
                 const int d = limh - c0;
                 uint32_t seen = 0;                // bit 16 cb + v: the cell of register v is visible
@@ -625,9 +626,9 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
                         const int off = 32 * cb + (v & 3) + 8 * (v >> 2);
                         const uint2 w = mv[4 * cb + (v >> 2)];
                         const uint32_t hw = (v & 2) ? w.y : w.x;
-                        const float x = mslope * f16_bits_to_float((uint16_t) (v & 1 ? hw >> 16 : hw));
+                        const float x = slope * f16_bits_to_float((uint16_t) (v & 1 ? hw >> 16 : hw));
                         const bool vis = off <= d && x != -AL_INF;
-                        sc[cb][v] = vis ? sc[cb][v] + x : -AL_INF;
+                        sc[cb][v] = vis ? __builtin_fmaf(sc[cb][v], snat, x) : -AL_INF;
                         seen |= vis ? 1u << (16 * cb + v) : 0u;
                     }
                 // by any row of the wave (the 32 lanes of a half hold the
@@ -693,14 +694,14 @@ __global__ __launch_bounds__(2 * kWaves * 64) void fattn_prefill_kernel(const Fa
         // of the wave sees counts as zeros (their probability of 0 times
         // whatever an unused cell holds).
         auto apply_gen = [&](const int i, const floatx16 (&sc)[2]) {
-            const float mc = m_run == -AL_INF ? 0.0f : m_run * cu;
+            const float mu = m_run == -AL_INF ? 0.0f : m_run;
             const bool drop = !__all(alive == ~0u);
             half8 pf[4];
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    pf[kk][e] = (_Float16) __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kk >> 1][8 * (kk & 1) + e], cu, -mc));
+                    pf[kk][e] = (_Float16) __builtin_amdgcn_exp2f((sc[kk >> 1][8 * (kk & 1) + e] - mu) * kLog2e);
 #pragma unroll
                 for (int e = 0; e < 8; e += 2)
                     l_run = __builtin_amdgcn_fdot2(half2v{pf[kk][e], pf[kk][e + 1]}, half2v{(_Float16) 1.0f, (_Float16) 1.0f}, l_run, false);

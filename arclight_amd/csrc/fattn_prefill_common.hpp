@@ -16,6 +16,7 @@ typedef float float2v __attribute__((ext_vector_type(2)));
 constexpr int kWaves = 4;                        // one per SIMD, 32 rows each
 constexpr int kLds = 160 * 1024;                 // the rings of all splits (all of a CU's LDS)
 constexpr float kLog2e = 1.44269504088896341f;
+constexpr float kLn2 = 0.693147180559945309f;
 
 __device__ __forceinline__ floatx16 mfma32(half8 a, half8 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);

@@ -721,3 +721,34 @@ def test_more_streams_than_the_decode_kernel_counts(gpu, G):
     sel = np.unique(np.concatenate([[0, 1, B - 1], rng.choice(B, 20, replace=False)]))
     assert_parity(got[sel], O.attention(np.ascontiguousarray(q[sel]), k, v, scale=SCALE, kv_len=n_kv - 3),
                   what=f"{G} heads to a kv head")
+
+
+@pytest.mark.parametrize("kw", [{}, {"max_bias": 8.0}, {"logit_softcap": 20.0}])
+@pytest.mark.parametrize("T,n_kv", [(9, 500), (16, 4096), (37, 3000), (256, 2048)])
+def test_masks_of_the_lowest_value(gpu, T, n_kv, kw):
+    """Tokens whose every cell has f16's lowest finite value for a mask: the
+    result is that of the scores alone, but for the sums' last bit, 1/256
+    beside 65504. The operator's definition, which the oracle restates, has
+    that rounding too; the kernel's splits add no other to it (their maxima
+    and weights are exact in these units): at most 1.25 of the oracle's
+    distance from 64 bits over a sample of heads."""
+    q, k, v = O.make_inputs(5 + T, T=T, Hq=32, Hkv=8, n_kv=n_kv)
+    m = O.causal_mask(T, n_kv, n_kv - T)
+    m[0, 0, 0] = -65504
+    m[0, 0, 2] = -65504
+    m[0, 0, 2, 100:200] = -np.inf
+    _case(f"{T} tokens over {n_kv} cells, two of the lowest mask value, {kw}")
+    got, ref = run_gpu(q, k, v, m, scale=SCALE, **kw), O.attention(q, k, v, m, scale=SCALE, **kw)
+    rest = [t for t in range(T) if t not in (0, 2)]
+    assert_parity(got[:, rest], ref[:, rest], what="the other tokens")
+    off, oracle = [], []
+    for t in (0, 2):
+        for h in range(0, 32, 2):
+            s = q[0, t, h].astype(np.float64) @ k[0, :, h // 4].astype(np.float64).T * SCALE
+            if "logit_softcap" in kw:
+                s = 20 * np.tanh(s / 20)
+            p = np.where(np.isneginf(m[0, 0, t]), 0.0, np.exp(s - s.max()))
+            exact = p @ v[0, :, h // 4].astype(np.float64) / p.sum()
+            off.append(got[0, t, h] - exact)
+            oracle.append(ref[0, t, h] - exact)
+    assert np.linalg.norm(off) <= 1.25 * np.linalg.norm(oracle), (np.linalg.norm(off), np.linalg.norm(oracle))
